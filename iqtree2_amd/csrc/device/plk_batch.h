@@ -19,7 +19,8 @@ struct BatchItem {
     InstDev I;
     ModelDev m;
     const plk_op* ops;     // this instance's ops inside the batch op array
-    const void* tables;    // [nops][2][table_size] storage precision
+    const void* tables;    // [nops][2][table_size] storage precision (4 states: and two steps more)
+    const TileOp* tops;    // 4 states: the ops as dna_ops reads them
     const double* root;    // val[C][n] then, for a tip dad, lut[SU+1][C][n]
     int nops;
     int table_size;
@@ -38,9 +39,18 @@ enum { BATCH_LNL = 0, BATCH_THETA = 1 };
 // staged in LDS once; row 0 also writes the item's root tables and workgroup
 // (0, 0) clears the work-list counters. LDS: evec n*n | tip SU*n | ex 2*C*n.
 template <typename T>
-__device__ inline void prep_child_table(const BatchItem& it, const plk_child ch, const double* ev_sh,
-                                        const double* tp_sh, const double* ex, T* out) {
+__device__ inline void prep_child_table(const BatchItem& it, const plk_child ch, int k, const double* ev_sh,
+                                        const double* tp_sh, const double* ex, T* step) {
     const int n = it.n, C = it.C, SU = it.I.SU, nn = n * n;
+    T* out = step + (size_t)k * it.table_size;
+    if (n == 4 && sizeof(T) == 8) {
+        for (int t = threadIdx.x; t < C * nn; t += kThreads) {
+            const int c = t / nn, r = t - c * nn;
+            const T v = (T)(ev_sh[r] * ex[c * n + r % n]);
+            dna_frag(C, c, r / n, r % n, k, [&](int at) { step[at] = v; });
+        }
+        return;
+    }
     if (!ch.is_tip) {
         if (n == kProtN) {
             // the matrix-core tile's fragment order
@@ -100,13 +110,17 @@ k_prep_batch(const BatchItem* __restrict__ items, const double* __restrict__ len
         }
         __syncthreads();
         for (int k = 0; k < 2; k++) {
-            const size_t off = (size_t)(2 * o + k) * it.table_size;
+            const size_t off = (size_t)2 * o * it.table_size;
+            void* tables = hbm(const_cast<void*>(it.tables));
             if (it.f32)
-                prep_child_table<float>(it, op.child[k], ev_sh, tp_sh, ex + k * nv,
-                                        reinterpret_cast<float*>(const_cast<void*>(it.tables)) + off);
+                prep_child_table<float>(it, op.child[k], k, ev_sh, tp_sh, ex + k * nv, reinterpret_cast<float*>(tables) + off);
             else
-                prep_child_table<double>(it, op.child[k], ev_sh, tp_sh, ex + k * nv,
-                                         reinterpret_cast<double*>(const_cast<void*>(it.tables)) + off);
+                prep_child_table<double>(it, op.child[k], k, ev_sh, tp_sh, ex + k * nv, reinterpret_cast<double*>(tables) + off);
+        }
+        if (n == 4 && threadIdx.x == 0) {
+            TileOp* tops = hbm(const_cast<TileOp*>(it.tops));
+            if (it.f32) make_tile_op<float>(it.I, it.ops, o, it.nops, tops);
+            else make_tile_op<double>(it.I, it.ops, o, it.nops, tops);
         }
     }
     if (blockIdx.y != 0) return;
@@ -186,10 +200,9 @@ __device__ inline double branch_end_stream(const InstDev& I, plk_end node, plk_e
 // 16-pattern MFMA sub-tiles of a protein batch tile
 constexpr int kBatchSub = 4;
 
-// Dynamic LDS bytes batch_tile uses for one item shape: U^-1, the two child
-// tables of a step and the root tables (which reuse the table area), or for
-// 20 states the maxima of prot_ops_tile (2 x kBatchSub x C x 16) and the
-// root tables.
+// Dynamic LDS bytes batch_tile uses for one item shape: what its op list needs
+// (4 states: dna_ops; 20 states: the maxima of prot_ops_tile, 2 x kBatchSub x
+// C x 16), then the root tables.
 __host__ __device__ inline size_t batch_smem_bytes(int n, int C, int SU, int table_size, size_t elem) {
     const size_t root = (size_t)(SU + 2) * n * C * 8;
     if (n == kCodonN) return (size_t)2 * n * kCodonStride * elem;   // E | U^-1; root rows stay in HBM
@@ -198,35 +211,26 @@ __host__ __device__ inline size_t batch_smem_bytes(int n, int C, int SU, int tab
         const size_t rt = (size_t)n * n * elem + root;
         return mf > rt ? mf : rt;
     }
-    const size_t tab = 2 * (size_t)table_size * elem;
-    return (size_t)n * n * elem + (tab > root ? tab : root);
+    const size_t ops = dna_ops_smem(SU);
+    return ops > root ? ops : root;
 }
 
-// patterns per thread of a 4-state batch tile: two, so that each step's
-// table staging and barriers serve twice the data and two patterns' loads
-// are in flight together
-constexpr int kDnaPatternsPerThread = 2;
-
-// patterns per work-list tile: 4 states, kDnaPatternsPerThread patterns per
-// C threads (128 with four categories); 20 and 61 states, one pattern per C
-// threads (four 16-pattern protein matrix-core tiles, or one codon tile)
-__host__ __device__ constexpr int batch_tile_patterns(int n, int C) {
-    return (n == 4 ? kDnaPatternsPerThread : 1) * kThreads / C;
-}
+// patterns per work-list tile: one per C threads (four 16-pattern protein
+// matrix-core tiles, one codon tile)
+__host__ __device__ constexpr int batch_tile_patterns(int C) { return kThreads / C; }
 
 // all ops of one tile of one item, then its root lnL; returns the tile's
 // lnL sum (thread 0)
 template <typename T, int N, int C>
 __device__ __forceinline__ double batch_tile(const BatchItem& it, int tile, unsigned char* smem) {
-    constexpr int PB = batch_tile_patterns(N, C);
-    constexpr int kPP = N == 4 ? kDnaPatternsPerThread : 1;   // patterns per thread
+    constexpr int PB = batch_tile_patterns(C);
     constexpr int block = N * C;
-    T* inv_sh = reinterpret_cast<T*>(smem);
-    T* tab_sh = inv_sh + N * N;
-    const InstDev& I = it.I;
+    const InstDev I = on_hbm(it.I);
+    const ModelDev m = on_hbm(it.m);
     const int c = threadIdx.x % C;
     const int p = tile * PB + (int)threadIdx.x / C;
-    const T* tables = reinterpret_cast<const T*>(it.tables);
+    const T* tables = hbm(reinterpret_cast<const T*>(it.tables));
+    const plk_op* ops = hbm(it.ops);
     __syncthreads();
     if constexpr (N == kCodonN) {
         // codon: the lone kernel's matrix-core tile, one pass per rate
@@ -235,44 +239,20 @@ __device__ __forceinline__ double batch_tile(const BatchItem& it, int tile, unsi
         static_assert(PB == kCodonTile, "batch tile must be one codon tile");
         T* e_m = reinterpret_cast<T*>(smem);
         T* inv_m = e_m + N * S;
-        stage_lds<N * N>(inv_m, it.m.inv_evec, N * N, [](int t) { return (t / N) * S + t % N; });
+        stage_lds<N * N>(inv_m, m.inv_evec, N * N, [](int t) { return (t / N) * S + t % N; });
         __syncthreads();
         for (int cc = 0; cc < C; cc++)
-            codon_ops_tile<T>(I, it.ops, it.nops, tables, it.table_size, cc, tile * PB, e_m, inv_m);
+            codon_ops_tile<T>(I, ops, it.nops, tables, it.table_size, cc, tile * PB, e_m, inv_m);
     } else if constexpr (N == 20) {
         // protein: the matrix-core tile of the lone traversal kernel, every
         // wave one category of four 16-pattern sub-tiles
         static_assert(PB == kBatchSub * kMfmaTile, "batch tile must be kBatchSub MFMA tiles");
-        prot_ops_tile<T, C, kBatchSub>(I, it.m.inv_evec, it.ops, it.nops, tables, it.table_size,
+        prot_ops_tile<T, C, kBatchSub>(I, m.inv_evec, ops, it.nops, tables, it.table_size,
                                        reinterpret_cast<T*>(smem), tile * PB);
     } else {
-    for (int t = threadIdx.x; t < N * N; t += kThreads) inv_sh[t] = (T)it.m.inv_evec[t];
-    for (int o = 0; o < it.nops; o++) {
-        const plk_op op = it.ops[o];
-        int left = 0, right = 1;
-        if (!op.child[0].is_tip && op.child[1].is_tip) { left = 1; right = 0; }
-        const plk_child L = op.child[left], R = op.child[right];
-        const int szL = L.is_tip ? (I.SU + 1) * block : block * N;
-        const int szR = R.is_tip ? (I.SU + 1) * block : block * N;
-        __syncthreads();
-        const T* gL = tables + (size_t)(2 * o + left) * it.table_size;
-        const T* gR = tables + (size_t)(2 * o + right) * it.table_size;
-        for (int t = threadIdx.x; t < szL; t += kThreads) tab_sh[t] = gL[t];
-        for (int t = threadIdx.x; t < szR; t += kThreads) tab_sh[it.table_size + t] = gR[t];
-        __syncthreads();
-        // the barrier above also orders the previous step's scale counters
-        // (written by the category-0 lane) before these loads
-        OpIn<T, N> in[kPP];
-#pragma unroll
-        for (int j = 0; j < kPP; j++)
-            op_load<T, N, C>(I, L.is_tip, L.id, R.is_tip, R.id, p + j * (kThreads / C), c, in[j]);
-#pragma unroll
-        for (int j = 0; j < kPP; j++)
-            op_finish<T, N, C>(I, inv_sh, tab_sh, tab_sh + it.table_size, L.is_tip, R.is_tip, op.dad_slot,
-                               p + j * (kThreads / C), c, in[j]);
+        dna_ops<T, C, false>(I, m, it.tops, it.nops, tables, it.table_size, tile * PB, reinterpret_cast<double*>(smem));
     }
-    }
-    double* root_sh = reinterpret_cast<double*>(tab_sh);
+    double* root_sh = reinterpret_cast<double*>(smem) + (N == kProtN ? N * N * sizeof(T) / 8 : 0);
     const plk_end node = it.node, dad = it.dad;
     __syncthreads();
     if (it.mode == BATCH_THETA) {
@@ -280,57 +260,52 @@ __device__ __forceinline__ double batch_tile(const BatchItem& it, int tile, unsi
         // (the streamed form reads them from HBM)
         if constexpr (N == 4) {
             if (dad.is_tip)
-                for (int t = threadIdx.x; t < (I.SU + 1) * N; t += kThreads) root_sh[t] = it.m.tip[t];
+                for (int t = threadIdx.x; t < (I.SU + 1) * N; t += kThreads) root_sh[t] = m.tip[t];
             __syncthreads();
-#pragma unroll
-            for (int j = 0; j < kPP; j++) theta_apply<T, N, C>(I, node, dad, root_sh, p + j * (kThreads / C), c);
+            theta_apply<T, N, C>(I, node, dad, root_sh, p, c);
         } else {
-            branch_end_stream<T, N, C>(I, node, dad, MODE_THETA, root_sh, p, c, it.m.tip);
+            branch_end_stream<T, N, C>(I, node, dad, MODE_THETA, root_sh, p, c, m.tip);
         }
         return 0.0;
     }
     if constexpr (N == kCodonN) {
         // 61-state lookup rows (121 KB for a tip dad) stay in HBM, as k_root_stream reads them
-        root_sh = const_cast<double*>(it.root);
+        root_sh = hbm(const_cast<double*>(it.root));
     } else {
         const int root_size = block + (dad.is_tip ? (I.SU + 1) * block : 0);
-        for (int t = threadIdx.x; t < root_size; t += kThreads) root_sh[t] = it.root[t];
+        for (int t = threadIdx.x; t < root_size; t += kThreads) root_sh[t] = hbm(it.root)[t];
         __syncthreads();
     }
     double contrib = 0.0;
+    double lh0;
+    int minsc;
+    if constexpr (N != 4) {
+        // streamed (no per-thread state arrays), same arithmetic as below
+        lh0 = branch_end_stream<T, N, C>(I, node, dad, MODE_BRANCH, root_sh, p, c, m.tip, &minsc);
+    } else {
+        double nv[N], dv[N], adjust;
+        load_branch<T, N, C>(I, node, dad, nullptr, p, c, nv, dv, minsc, adjust);
+        double lhc;
+        if (dad.is_tip) {
+            const int s = I.states[(size_t)dad.id * I.Ppad + p];
+            const double* lut = root_sh + block + (s * C + c) * N;
+            lhc = lut[0] * nv[0];
 #pragma unroll
-    for (int j = 0; j < kPP; j++) {
-        const int pj = p + j * (kThreads / C);
-        double lh0;
-        int minsc;
-        if constexpr (N != 4) {
-            // streamed (no per-thread state arrays), same arithmetic as below
-            lh0 = branch_end_stream<T, N, C>(I, node, dad, MODE_BRANCH, root_sh, pj, c, it.m.tip, &minsc);
+            for (int i = 1; i < N; i++) lhc = fma(lut[i], nv[i], lhc);
         } else {
-            double nv[N], dv[N], adjust;
-            load_branch<T, N, C>(I, node, dad, nullptr, pj, c, nv, dv, minsc, adjust);
-            double lhc;
-            if (dad.is_tip) {
-                const int s = I.states[(size_t)dad.id * I.Ppad + pj];
-                const double* lut = root_sh + block + (s * C + c) * N;
-                lhc = lut[0] * nv[0];
+            const double* val = root_sh + c * N;
+            lhc = val[0] * dv[0] * nv[0];
 #pragma unroll
-                for (int i = 1; i < N; i++) lhc = fma(lut[i], nv[i], lhc);
-            } else {
-                const double* val = root_sh + c * N;
-                lhc = val[0] * dv[0] * nv[0];
-#pragma unroll
-                for (int i = 1; i < N; i++) lhc = fma(val[i] * dv[i], nv[i], lhc);
-            }
-            lh0 = I.safe ? group_sum_sumvec<C>(lhc * adjust) : group_sum_ordered<C>(lhc);
+            for (int i = 1; i < N; i++) lhc = fma(val[i] * dv[i], nv[i], lhc);
         }
-        if (c == 0) {
-            const double lh = fabs(lh0) + I.invar[pj];
-            const double lnp = log(lh) + (double)minsc * Prec<T>::log_unit;
-            if (pj < I.P) {
-                I.ptn_lh[pj] = lnp;
-                contrib += lnp * I.freq[pj];
-            }
+        lh0 = I.safe ? group_sum_sumvec<C>(lhc * adjust) : group_sum_ordered<C>(lhc);
+    }
+    if (c == 0) {
+        const double lh = fabs(lh0) + I.invar[p];
+        const double lnp = log(lh) + (double)minsc * Prec<T>::log_unit;
+        if (p < I.P) {
+            I.ptn_lh[p] = lnp;
+            contrib = lnp * I.freq[p];
         }
     }
     double v[1] = {contrib};
@@ -373,7 +348,7 @@ struct XcdSplit {
 // own choice left each one wave lower.
 template <int MASK>
 __global__ void __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(MASK == BC_PROT64 ? 3 : (MASK == BC_PROT32 ? 4 : 1))))
+__attribute__((amdgpu_waves_per_eu(MASK == BC_PROT64 ? 3 : (MASK == BC_PROT32 || MASK == BC_DNA64 || MASK == BC_DNA32 ? 4 : 1))))
 k_batch(const BatchItem* __restrict__ items, const int* __restrict__ tile_item, XcdSplit xs,
         unsigned* __restrict__ counters, double* __restrict__ tile_sums) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -453,7 +428,7 @@ k_derv_batch(const DervItem* __restrict__ items, const int* __restrict__ tile_it
     __shared__ double red[3 * (kThreads / 64)];
     const int g = tile_begin + blockIdx.x;
     const DervItem& it = items[tile_item[g]];
-    buffer_block<T, N, C>(it.I, it.m, it.length, BUF_DERV, g - it.tile_begin, val, red,
+    buffer_block<T, N, C>(on_hbm(it.I), on_hbm(it.m), it.length, BUF_DERV, g - it.tile_begin, val, red,
                           tile_sums + 3 * (size_t)g);
 }
 

@@ -88,6 +88,7 @@ struct Instance {
     size_t elem = 8;            // bytes of one stored value
     size_t scale_elem = 2;      // bytes of one scale counter
     int table_size = 0;         // elements per (op, child) table
+    int chunk_slots = 0;        // slots of a chunk (Part)
     int sweep_table_size = 0;   // elements per child table in the sweep's LDS layout
     size_t bytes = 0;           // HBM held
     // device buffers
@@ -124,6 +125,7 @@ struct Instance {
     unsigned char* sw_tabs = nullptr; // codon sweep: two steps' child tables
     size_t sw_tabs_cap = 0;
     void* tables = nullptr;
+    TileOp* tops = nullptr;           // 4 states: the staged ops as dna_ops reads them
     bool patterns_set = false, model_set = false, theta_ready = false, ptn_lh_ready = false;
     double theta_length = 0.0;
     // Fitch parsimony state (allocated by the first parsimony call)
@@ -160,6 +162,10 @@ struct Instance {
 
 size_t alloc_class(size_t bytes);
 
+// slots the arrays hold: 4 states an odd number; and counters of a pattern (Part)
+int stored_slots(const plk_instance_desc* d) { return d->nstates == 4 ? d->nslots | 1 : d->nslots; }
+int stored_counts(const plk_instance_desc* d) { return d->safe_numeric || d->nstates == 4 ? d->ncat : 1; }
+
 // red_out: 8 reduced scalars, then four values per unobserved pattern of
 // +ASC when there are at most kAscMax of them (the constant patterns of
 // ASC_VARIANT, one per state); the larger sets of ASC_INFORMATIVE live in
@@ -174,24 +180,26 @@ size_t footprint_of(const plk_instance_desc* d, int Ppad) {
     const size_t scale_elem = d->precision == PLK_PREC_F32 ? 4 : 2;
     const size_t n = d->nstates, SU = d->state_unknown;
     const size_t block = n * d->ncat;
-    const size_t ncnt = d->safe_numeric ? d->ncat : 1;
-    const size_t table = std::max(block * n, (SU + 1) * block);
+    const size_t ncnt = stored_counts(d);
+    const size_t table = n == 4 ? dna_table_size(d->ncat, d->state_unknown, elem) : std::max(block * n, (SU + 1) * block);
     const size_t bufs[] = {
         (size_t)d->ntaxa * Ppad,                                  // states
         (size_t)Ppad * 8, (size_t)Ppad * 8,                       // freq, invar
         (n + 2 * n * n + (SU + 1) * n + 2 * (size_t)d->ncat) * 8, // model
-        (size_t)d->nslots * Ppad * block * elem,                  // partials
-        (size_t)d->nslots * Ppad * ncnt * scale_elem,             // scale counters
+        (size_t)stored_slots(d) * Ppad * block * elem,            // partials
+        (size_t)stored_slots(d) * Ppad * ncnt * scale_elem,       // scale counters
         (size_t)Ppad * block * elem,                              // theta
         (size_t)Ppad * 8, (size_t)Ppad * 8,                       // buffer_scale, ptn_lh
         (size_t)(Ppad / (kThreads / 8) + 1) * 3 * 8,              // block sums
         kRedOutDoubles * 8,                                       // reduced scalars, +ASC values
         (SU + 2) * block * 8,                                     // root tables
         sizeof(plk_op) * (size_t)d->nslots,                       // ops of a full traversal
-        (size_t)d->nslots * 2 * table * elem,                     // and their tables
+        (size_t)(d->nslots + 2) * 2 * table * elem,               // and their tables
+        d->nstates == 4 ? sizeof(TileOp) * (size_t)(d->nslots + kTileAhead) : 0,
     };
     size_t b = 0;
-    for (size_t x : bufs) b += alloc_class(x);
+    for (size_t x : bufs)
+        if (x) b += alloc_class(x);
     return b;
 }
 
@@ -360,7 +368,7 @@ plk_status destroy_instance(plk_context* ctx, int id) {
     if (!in) return fail(PLK_ERR_ARG, "unknown instance %d", id);
     void* bufs[] = {in->states, in->freq, in->invar, in->model, in->partial, in->scale,
                     in->theta, in->buffer_scale, in->ptn_lh, in->block_sums, in->red_out,
-                    in->root_tab, in->ops, in->tables, in->sw_ops, in->sw_br, in->sw_len,
+                    in->root_tab, in->ops, in->tables, in->tops, in->sw_ops, in->sw_br, in->sw_len,
                     in->sw_nderv, in->sw_part, in->sw_flags, in->sw_out, in->sw_timing, in->sw_res, in->sw_tabs,
                     in->pars_tip_planes, in->pars_planes, in->pars_counts, in->pars_sets,
                     in->pars_changes, in->pars_ops, in->asc_vals, in->nr_model, in->nr_root,
@@ -427,9 +435,28 @@ InstDev inst_dev(const Instance* in) {
     I.ptn_lh = in->ptn_lh;
     I.slot_stride = (size_t)in->Ppad * in->block;
     I.scale_stride = (size_t)in->Ppad * (in->d.safe_numeric ? in->d.ncat : 1);
+    I.chunk_slots = in->chunk_slots;
     I.nasc = in->nasc;
     I.asc = in->nasc > kAscMax ? in->asc_vals : in->red_out + 8;
     return I;
+}
+
+// where an instance's own shape keeps a slot's values and counters (Part)
+struct Places {
+    size_t at, by, count;
+};
+template <typename T>
+Places places_of(const Instance* in, int slot, int p, int c) {
+    const InstDev I = inst_dev(in);
+    auto put = [&](auto part) { return Places{part.at(I, slot, p, c), (size_t)part.stride, part.count_at(I, slot, p, c)}; };
+    if (in->d.nstates == 4) switch (in->d.ncat) {
+        case 1: return put(Part<T, 4, 1>());
+        case 2: return put(Part<T, 4, 2>());
+        case 4: return put(Part<T, 4, 4>());
+        case 8: return put(Part<T, 4, 8>());
+        }
+    const size_t pc = (size_t)p * in->d.ncat + c;
+    return Places{slot * I.slot_stride + pc * in->d.nstates, 1, slot * I.scale_stride + (in->d.safe_numeric ? pc : (size_t)p)};
 }
 
 ModelDev model_dev(const Instance* in) {
@@ -506,15 +533,17 @@ plk_status launch_traverse_t(plk_context* ctx, Instance* in, int nops, int mode,
                              plk_end dad) {
     const int PB = kThreads / C;
     const int grid = in->Ppad / PB;
-    const size_t tab_bytes = 2 * (size_t)in->table_size * sizeof(T);
-    const size_t root_bytes = (size_t)(in->d.state_unknown + 2) * in->block * 8;
-    const size_t smem = round_up((size_t)N * N * sizeof(T), 16) + std::max(tab_bytes, root_bytes);
+    // the tip vectors, then the root stage's tables
+    const size_t smem = std::max(dna_ops_smem(in->d.state_unknown), (size_t)(in->d.state_unknown + 2) * in->block * 8);
     if (smem > 160 * 1024) return fail(PLK_ERR_UNSUPPORTED, "LDS need %zu bytes", smem);
     const int pe = prof_begin(ctx);
-    hipLaunchKernelGGL((k_traverse<T, N, C>), dim3(grid), dim3(kThreads), smem, ctx->stream,
-                       inst_dev(in), model_dev(in), in->ops, nops,
-                       reinterpret_cast<const T*>(in->tables), in->table_size, mode, node, dad,
-                       in->root_tab, in->block_sums);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), smem, ctx->stream, inst_dev(in), model_dev(in), in->tops,
+                           nops, reinterpret_cast<const T*>(in->tables), in->table_size, mode, node, dad,
+                           in->root_tab, in->block_sums);
+    };
+    if (dna_far(in->chunk_slots, sizeof(T))) go(k_traverse<T, N, C, true>);
+    else go(k_traverse<T, N, C, false>);
     HIP_TRY(hipGetLastError());
     if (pe >= 0) {
         const double P = in->d.npatterns, s = (double)in->elem, blk = (double)in->block;
@@ -717,13 +746,16 @@ plk_status stage_ops(plk_context* ctx, Instance* in, const plk_op* ops, int nops
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         dfree(ctx, in, in->ops, sizeof(plk_op) * in->ops_cap);
         dfree(ctx, in, in->tables, (size_t)in->ops_cap * 2 * in->table_size * elem);
+        dfree(ctx, in, in->tops, sizeof(TileOp) * in->ops_cap);
         in->ops = nullptr;
         in->tables = nullptr;
+        in->tops = nullptr;
         const int cap = std::max(nops, 2 * in->ops_cap);
         st = dmalloc(ctx, in, &in->ops, sizeof(plk_op) * cap);
         if (st != PLK_OK) return st;
-        st = dmalloc(ctx, in, &in->tables, (size_t)cap * 2 * in->table_size * elem);
+        st = dmalloc(ctx, in, &in->tables, (size_t)(cap + 2) * 2 * in->table_size * elem);   // dna_ops reads two steps on
         if (st != PLK_OK) return st;
+        if (in->d.nstates == 4 && (st = dmalloc(ctx, in, &in->tops, sizeof(TileOp) * (cap + kTileAhead))) != PLK_OK) return st;
         in->ops_cap = cap;
     }
     std::vector<plk_op> stripped;
@@ -761,20 +793,22 @@ plk_status stage_ops(plk_context* ctx, Instance* in, const plk_op* ops, int nops
         if (in->d.precision == PLK_PREC_F32) {
             hipLaunchKernelGGL(k_nr_prep_ops<float>, grid, dim3(kThreads), nsmem, ctx->stream, in->ops,
                                in->nr_flags, nops, nr_dev(in), tip, in->d.state_unknown, in->table_size,
-                               reinterpret_cast<float*>(in->tables));
+                               reinterpret_cast<float*>(in->tables), inst_dev(in), in->tops);
         } else {
             hipLaunchKernelGGL(k_nr_prep_ops<double>, grid, dim3(kThreads), nsmem, ctx->stream, in->ops,
                                in->nr_flags, nops, nr_dev(in), tip, in->d.state_unknown, in->table_size,
-                               reinterpret_cast<double*>(in->tables));
+                               reinterpret_cast<double*>(in->tables), inst_dev(in), in->tops);
         }
     } else if (in->d.precision == PLK_PREC_F32) {
         hipLaunchKernelGGL(k_prep_ops<float>, grid, dim3(kThreads), smem, ctx->stream,
                            in->ops, nops, model_dev(in), in->d.nstates, in->d.ncat,
-                           in->d.state_unknown, in->table_size, reinterpret_cast<float*>(in->tables));
+                           in->d.state_unknown, in->table_size, reinterpret_cast<float*>(in->tables),
+                           inst_dev(in), in->tops);
     } else {
         hipLaunchKernelGGL(k_prep_ops<double>, grid, dim3(kThreads), smem, ctx->stream,
                            in->ops, nops, model_dev(in), in->d.nstates, in->d.ncat,
-                           in->d.state_unknown, in->table_size, reinterpret_cast<double*>(in->tables));
+                           in->d.state_unknown, in->table_size, reinterpret_cast<double*>(in->tables),
+                           inst_dev(in), in->tops);
     }
     HIP_TRY(hipGetLastError());
     prof_end(ctx, pe, K_PREP_OPS, 2.0 * nops * in->table_size * in->elem, 0.0);
@@ -1091,12 +1125,15 @@ plk_status plk_instance_create(plk_context* ctx, const plk_instance_desc* d, int
     in->d = *d;
     in->Ppad = Ppad;
     in->block = (size_t)d->nstates * d->ncat;
+    in->chunk_slots = stored_slots(d);
     in->elem = d->precision == PLK_PREC_F32 ? 4 : 8;
     in->scale_elem = d->precision == PLK_PREC_F32 ? 4 : 2;
     in->sweep_table_size = (int)std::max(in->block * d->nstates, (size_t)(d->state_unknown + 1) * in->block);
-    in->table_size = d->nstates == kProtN ? prot_table_size(d->ncat, d->state_unknown) : in->sweep_table_size;
+    in->table_size = d->nstates == kProtN ? prot_table_size(d->ncat, d->state_unknown)
+                     : d->nstates == 4  ? dna_table_size(d->ncat, d->state_unknown, in->elem)
+                                        : in->sweep_table_size;
     const int n = d->nstates;
-    const size_t ncnt = d->safe_numeric ? d->ncat : 1;
+    const size_t ncnt = stored_counts(d);
     const size_t model_doubles = n + 2 * (size_t)n * n + (size_t)(d->state_unknown + 1) * n + 2 * d->ncat;
     const int max_grid = Ppad / (kThreads / 8) + 1;
     plk_status st = PLK_OK;
@@ -1107,8 +1144,8 @@ plk_status plk_instance_create(plk_context* ctx, const plk_instance_desc* d, int
     A(&in->freq, (size_t)Ppad * 8);
     A(&in->invar, (size_t)Ppad * 8);
     A(&in->model, model_doubles * 8);
-    A(&in->partial, (size_t)d->nslots * Ppad * in->block * in->elem);
-    A(&in->scale, (size_t)d->nslots * Ppad * ncnt * in->scale_elem);
+    A(&in->partial, (size_t)in->chunk_slots * Ppad * in->block * in->elem);
+    A(&in->scale, (size_t)in->chunk_slots * Ppad * ncnt * in->scale_elem);
     A(&in->theta, (size_t)Ppad * in->block * in->elem);
     A(&in->buffer_scale, (size_t)Ppad * 8);
     A(&in->ptn_lh, (size_t)Ppad * 8);
@@ -1120,7 +1157,7 @@ plk_status plk_instance_create(plk_context* ctx, const plk_instance_desc* d, int
         if (hipMemsetAsync(in->states, d->state_unknown, (size_t)d->ntaxa * Ppad, ctx->stream) != hipSuccess ||
             hipMemsetAsync(in->freq, 0, (size_t)Ppad * 8, ctx->stream) != hipSuccess ||
             hipMemsetAsync(in->invar, 0, (size_t)Ppad * 8, ctx->stream) != hipSuccess ||
-            hipMemsetAsync(in->scale, 0, (size_t)d->nslots * Ppad * ncnt * in->scale_elem, ctx->stream) != hipSuccess ||
+            hipMemsetAsync(in->scale, 0, (size_t)in->chunk_slots * Ppad * ncnt * in->scale_elem, ctx->stream) != hipSuccess ||
             hipStreamSynchronize(ctx->stream) != hipSuccess)
             st = fail(PLK_ERR_DEVICE, "initialising instance buffers failed");
     }
@@ -1663,7 +1700,7 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
         const double n = in->d.nstates;
         cost[i] = (double)in->d.npatterns * (items[i].nops + 1) * n * n;
         cls[i] = batch_class(in->d.nstates, in->d.precision == PLK_PREC_F32);
-        const int PB = batch_tile_patterns(in->d.nstates, in->d.ncat);
+        const int PB = batch_tile_patterns(in->d.ncat);
         ntiles_of[i] = (in->d.npatterns + PB - 1) / PB;
         total_tiles += ntiles_of[i];
         if (!(mix & cls[i])) nclasses++;
@@ -1760,7 +1797,7 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
         op_off[r] = nops_total;
         nops_total += items[i].nops;
         max_nops = std::max(max_nops, items[i].nops);
-        const int PB = batch_tile_patterns(in->d.nstates, in->d.ncat);
+        const int PB = batch_tile_patterns(in->d.ncat);
         BatchItem& b = hb[r];
         b.I = inst_dev(in);
         b.m = model_dev(in);
@@ -1776,7 +1813,9 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
         b.mode = modes ? modes[i] : BATCH_LNL;
         tiles_so_far += b.ntiles;
         b.tables = reinterpret_cast<const void*>(tab_bytes);   // offsets until the buffers exist
-        tab_bytes += round_up((size_t)items[i].nops * 2 * in->table_size * in->elem, 256);
+        tab_bytes += round_up((size_t)(items[i].nops + (b.n == 4 ? 2 : 0)) * 2 * in->table_size * in->elem, 256);
+        b.tops = reinterpret_cast<const TileOp*>(tab_bytes);
+        if (b.n == 4) tab_bytes += round_up(sizeof(TileOp) * (size_t)(items[i].nops + kTileAhead), 256);
         b.root = reinterpret_cast<const double*>(root_doubles);
         root_doubles += (size_t)(in->d.state_unknown + 2) * in->block;
         const size_t item_smem = batch_smem_bytes(b.n, b.C, in->d.state_unknown, in->table_size, in->elem);
@@ -1821,6 +1860,7 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
         BatchItem& b = hb[r];
         b.ops = d_ops + op_off[r];
         b.tables = ctx->bt_tables + reinterpret_cast<size_t>(b.tables);
+        b.tops = reinterpret_cast<const TileOp*>(ctx->bt_tables + reinterpret_cast<size_t>(b.tops));
         b.root = ctx->bt_roots + reinterpret_cast<size_t>(b.root);
         if (items[i].nops) std::memcpy(h_ops + op_off[r], items[i].ops, sizeof(plk_op) * items[i].nops);
         for (int t = 0; t < b.ntiles; t++) h_tiles[b.tile_begin + t] = r;
@@ -1974,7 +2014,7 @@ plk_status plk_batch_evaluate(plk_context* ctx, const plk_batch_item* items, con
     bool nonfinite = false;
     for (int i = 0; i < nitems; i++) {
         const Instance* in = ins[i];
-        if (in->d.ncat == 4 && in->nasc == 0 && !in->nonrev &&
+        if (in->d.ncat == 4 && in->nasc == 0 && !in->nonrev && !(in->d.nstates == 4 && dna_far(in->chunk_slots, in->elem)) &&
             (in->d.nstates == 4 || in->d.nstates == 20 || in->d.nstates == kCodonN)) {
             fused.push_back(items[i]);
             fused_ins.push_back(ins[i]);
@@ -2699,30 +2739,39 @@ plk_status plk_read_partial(plk_context* ctx, int id, int slot, double* partial,
     if (!in) return fail(PLK_ERR_ARG, "unknown instance");
     if (slot < 0 || slot >= in->d.nslots) return fail(PLK_ERR_ARG, "slot out of range");
     std::lock_guard<std::mutex> lock(ctx->mu);
-    const int P = in->d.npatterns;
-    const size_t ncnt = in->d.safe_numeric ? in->d.ncat : 1;
-    if (partial) {
-        const size_t cnt = (size_t)P * in->block;
-        std::vector<unsigned char> h(cnt * in->elem);
-        const unsigned char* src = reinterpret_cast<const unsigned char*>(in->partial) +
-                                   (size_t)slot * in->Ppad * in->block * in->elem;
-        HIP_TRY(hipMemcpyAsync(h.data(), src, h.size(), hipMemcpyDeviceToHost, ctx->stream));
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
-        for (size_t i = 0; i < cnt; i++)
-            partial[i] = in->elem == 8 ? reinterpret_cast<const double*>(h.data())[i]
-                                       : (double)reinterpret_cast<const float*>(h.data())[i];
-    }
-    if (scale) {
-        const size_t cnt = (size_t)P * ncnt;
-        std::vector<unsigned char> h(cnt * in->scale_elem);
-        const unsigned char* src = reinterpret_cast<const unsigned char*>(in->scale) +
-                                   (size_t)slot * in->Ppad * ncnt * in->scale_elem;
-        HIP_TRY(hipMemcpyAsync(h.data(), src, h.size(), hipMemcpyDeviceToHost, ctx->stream));
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
-        for (size_t i = 0; i < cnt; i++)
-            scale[i] = in->scale_elem == 2 ? (int32_t)reinterpret_cast<const uint16_t*>(h.data())[i]
-                                           : reinterpret_cast<const int32_t*>(h.data())[i];
-    }
+    const int P = in->d.npatterns, n = in->d.nstates, C = in->d.ncat;
+    // a slot's values and counters as stored: one stretch of each, or for 4
+    // states one of each chunk
+    const int chunks = n == 4 ? in->Ppad * C / 64 : 1;
+    const size_t ncnt = in->d.safe_numeric ? C : 1;
+    const size_t vb = (size_t)in->Ppad * in->block * in->elem / chunks, cb = (size_t)in->Ppad * stored_counts(&in->d) * in->scale_elem / chunks;
+    std::vector<unsigned char> hv(partial ? vb * chunks : 0), hc(scale ? cb * chunks : 0);
+    auto fetch = [&](std::vector<unsigned char>& h, const void* src, size_t bytes) -> plk_status {
+        if (h.empty()) return PLK_OK;
+        const unsigned char* from = reinterpret_cast<const unsigned char*>(src) + (size_t)slot * bytes;
+        HIP_TRY(hipMemcpy2DAsync(h.data(), bytes, from, (size_t)in->chunk_slots * bytes, bytes, chunks,
+                                 hipMemcpyDeviceToHost, ctx->stream));
+        return PLK_OK;
+    };
+    plk_status st;
+    if ((st = fetch(hv, in->partial, vb)) != PLK_OK) return st;
+    if ((st = fetch(hc, in->scale, cb)) != PLK_OK) return st;
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    // the copies hold this slot alone: places of an instance of one slot
+    Instance one = *in;
+    one.chunk_slots = 1;
+    const bool f64 = in->elem == 8;
+    for (int p = 0; p < P; p++)
+        for (int c = 0; c < C; c++) {
+            const Places at = f64 ? places_of<double>(&one, 0, p, c) : places_of<float>(&one, 0, p, c);
+            if (partial)
+                for (int x = 0; x < n; x++)
+                    *partial++ = f64 ? reinterpret_cast<const double*>(hv.data())[at.at + x * at.by]
+                                     : (double)reinterpret_cast<const float*>(hv.data())[at.at + x * at.by];
+            if (scale && (c == 0 || ncnt > 1))
+                *scale++ = in->scale_elem == 2 ? (int32_t)reinterpret_cast<const uint16_t*>(hc.data())[at.count]
+                                               : reinterpret_cast<const int32_t*>(hc.data())[at.count];
+        }
     return PLK_OK;
 }
 

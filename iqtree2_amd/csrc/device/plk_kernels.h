@@ -1,15 +1,15 @@
 // HIP kernels of the likelihood engine (gfx950, wave64).
 //
 // Layout in HBM (one instance):
-//   partial[slot][p][c][x]   T (double or float), pattern-major, eigen basis
+//   partial[slot][p][c][x]   T (double or float), pattern-major, eigen basis;
+//                            4 states: in chunks of 64 pairs, Part below
 //   scale[slot][p]           uint16 (FP64 form) / int32 exponent (FP32 form),
-//                            [slot][p][c] in safe mode
+//                            [slot][p][c] in safe mode; 4 states as Part says
 //   theta[p][c][x]           T; buffer_scale[p] double
 //   states[taxon][p]         uint8
 // Thread mapping: one thread per (pattern, category); the C threads of a
-// pattern are adjacent lanes of one wavefront, so a pattern's block of C*n
-// values is read and written as one contiguous run, and cross-category
-// reductions are lane shuffles. A workgroup owns a tile of 256/C patterns
+// pattern are adjacent lanes of one wavefront, so cross-category reductions are
+// lane shuffles. A workgroup owns a tile of 256/C patterns
 // and walks the whole post-order op list for that tile: patterns are
 // independent, so no synchronisation crosses workgroups.
 #pragma once
@@ -83,12 +83,91 @@ struct InstDev {
     double* ptn_lh;          // [Ppad]
     size_t slot_stride;      // Ppad*block
     size_t scale_stride;     // Ppad*(safe?C:1)
+    int chunk_slots;         // 4 states: slots of a chunk (Part)
     // +ASC (Lewis): the last nasc of the P patterns are the unobserved
     // constant patterns; pattern k's lh goes to asc[4k], and a derivative
     // evaluation adds lh as the derivative sum counts it, d1 and d2 at 4k+1..3
     int nasc;
     double* asc;
 };
+
+// A pointer that was itself read from memory has no address space, and every
+// access through it is a flat one (through the LDS aperture check, waiting for
+// LDS and memory alike). hbm(p) makes it one to device memory.
+template <typename T>
+using Hbm = __attribute__((address_space(1))) T;
+template <typename T>
+__device__ inline T* hbm(T* p) { return (T*)(Hbm<T>*)(uint64_t)p; }
+__device__ inline void* hbm(void* p) { return (void*)(Hbm<char>*)(uint64_t)p; }
+__device__ inline InstDev on_hbm(InstDev I) {
+    I.states = hbm(I.states);
+    I.freq = hbm(I.freq);
+    I.invar = hbm(I.invar);
+    I.partial = hbm(I.partial);
+    I.scale = hbm(I.scale);
+    I.theta = hbm(I.theta);
+    I.buffer_scale = hbm(I.buffer_scale);
+    I.ptn_lh = hbm(I.ptn_lh);
+    I.asc = hbm(I.asc);
+    return I;
+}
+__device__ inline ModelDev on_hbm(ModelDev m) {
+    return ModelDev{hbm(m.eval), hbm(m.evec), hbm(m.inv_evec), hbm(m.tip), hbm(m.rates), hbm(m.props)};
+}
+
+// Where slot s keeps value x of (pattern p, category c), element
+// at(I, s, p, c) + x * stride, and its counter, element count_at(I, s, p, c)
+// ([slot][p], safe mode [slot][p][c]; 4 states one per pair in both modes, so
+// that a wavefront writes whole lines).
+// 4 states: 64 (pattern, category) pairs, those of 64 / C adjacent patterns,
+// make a chunk, and a chunk keeps all its slots together, so that the
+// wavefront that walks a tree for it (dna_ops) stays in one stretch of memory
+// and addresses it by 32-bit offsets. A chunk has an odd number of slots:
+// wavefronts that write the same slot at a time then spread over the memory
+// channels (200 taxa x 100,000 sites, even: 1,042 us, odd: 1,031). In a chunk's slot, four patterns' pairs
+// of a category are adjacent: pair (p / 4, c, p % 4), and pair l's values are
+//   float    at 4l + x
+//   double   at [g / 2][x][j][g % 2] of pair l = j + 16g (j < 16): a lane's
+//            matrix operands, sixteen bytes at a time
+template <typename T, int N, int C>
+struct Part {
+    static constexpr bool kLanes = N == 4 && sizeof(T) == 8;
+    static constexpr int stride = kLanes ? 32 : 1;
+    __host__ __device__ static size_t at(const InstDev& I, int slot, int p, int c) {
+        if (N != 4) return slot * I.slot_stride + (size_t)p * (N * C) + c * N;
+        const int l = pair(p, c);
+        const int in = kLanes ? (l >> 5) * 128 + (l & 15) * 2 + (l >> 4 & 1) : l * 4;
+        return ((size_t)(p / (64 / C)) * I.chunk_slots + slot) * 256 + in;
+    }
+    __host__ __device__ static size_t count_at(const InstDev& I, int slot, int p, int c) {
+        if (N != 4) return slot * I.scale_stride + (I.safe ? (size_t)p * C + c : (size_t)p);
+        return ((size_t)(p / (64 / C)) * I.chunk_slots + slot) * 64 + pair(p, c);
+    }
+    __host__ __device__ static int pair(int p, int c) { return (p % (64 / C) >> 2) * (4 * C) + 4 * c + (p & 3); }
+    // the thread of (p, c) writes a counter of its own
+    __device__ static bool counts(const InstDev& I, int c) { return N == 4 || I.safe || c == 0; }
+};
+
+// Elements of one (op, child) table for 4 states. Double storage: a child's
+// matrices, a tip's too (its product with the tip vectors is part of the step,
+// dna_ops), as operands of the matrix products: lane l's elements of a step,
+// child 0's then child 1's, are adjacent (dna_frag). Float storage: an internal
+// child's matrices [C][4][4], a tip child's lookup [SU+1][C][4], whose product
+// is rounded once.
+__host__ __device__ inline int dna_table_size(int C, int SU, size_t elem) {
+    const int mat = C == 8 ? 128 : 64, lut = (SU + 1) * C * 4;
+    return elem == 8 ? mat : lut > C * 16 ? lut : C * 16;
+}
+// where element (x, i) of category c's matrix of child k goes among a step's
+// 2 * dna_table_size elements: f(place) for each copy
+template <typename F>
+__device__ inline void dna_frag(int C, int c, int x, int i, int k, F f) {
+    for (int b = 0; b < 4; b++)
+        for (int h = 0; h < (C == 8 ? 2 : 1); h++) {
+            const int cat = C == 1 ? 0 : C == 2 ? b & 1 : C == 4 ? b : b + 4 * h;
+            if (cat == c) f(128 * h + 2 * (x + 4 * b + 16 * i) + k);
+        }
+}
 
 // Transition tables of protein (20-state) internal children are stored in
 // the operand order of the matrix-core tile (plk_mfma.h).
@@ -125,27 +204,77 @@ k_copy(const double4* __restrict__ src, double4* __restrict__ dst, size_t n) {
 enum TraverseMode { MODE_PARTIALS = 0, MODE_BRANCH = 1, MODE_THETA = 2 };
 enum BufferMode { BUF_DERV = 0, BUF_LNL = 1 };
 
+// One traversal step for dna_ops (4 states): three scalar loads of sixteen
+// bytes, each made when its part of the step is due.
+struct alignas(64) TileOp {
+    uint64_t tip[2];      // a tip child's row of states (others: taxon 0's)
+    uint32_t v[2], sc[2]; // a slot child's values and counters, kNoSlot for one that comes from elsewhere
+    uint32_t dst, dsc;    // the dad's; offsets in bytes from the chunk's slot 0 (far instances: slots)
+    uint32_t kind;        // of child k in bits 2k and 2k + 1, below
+    uint32_t root;        // bit k: child k is the root leaf (state-basis models)
+};
+// a slot in memory, the dad of the step before (in registers), the dad of the
+// step before that, a tip
+enum TileChild { CHILD_SLOT = 0, CHILD_LAST = 1, CHILD_LAST2 = 2, CHILD_TIP = 3 };
+constexpr uint32_t kNoSlot = 0xFFFFF800u;    // past the end of a chunk's buffer
+constexpr int kTileAhead = 6;                // steps that dna_ops looks ahead: copies of the last TileOp
+
+// bytes of a chunk's slot: values, counters
+template <typename T> constexpr uint32_t kChunkValues = 256 * sizeof(T);
+template <typename T> constexpr uint32_t kChunkCounts = 64 * sizeof(typename Prec<T>::scale_t);
+// a chunk of more slots than 32-bit offsets reach (two million in double storage)
+__host__ __device__ inline bool dna_far(int chunk_slots, size_t elem) {
+    return (uint64_t)chunk_slots * 256 * elem > kNoSlot;
+}
+
+// steps nops .. nops + kTileAhead - 1 repeat the last
+template <typename T>
+__device__ inline void make_tile_op(const InstDev& I, const plk_op* __restrict__ ops, int o, int nops, TileOp* tops,
+                                    unsigned root = 0) {
+    const plk_op op = ops[o];
+    const int last = o > 0 ? ops[o - 1].dad_slot : -1, last2 = o > 1 ? ops[o - 2].dad_slot : -1;
+    const bool far = dna_far(I.chunk_slots, sizeof(T));
+    const uint32_t nv = far ? 1 : kChunkValues<T>, nc = far ? 1 : kChunkCounts<T>;
+    TileOp t;
+    t.kind = 0;
+    for (int k = 0; k < 2; k++) {
+        const int id = op.child[k].id;
+        const int kind = op.child[k].is_tip ? CHILD_TIP : id == last ? CHILD_LAST : id == last2 ? CHILD_LAST2 : CHILD_SLOT;
+        t.kind |= kind << 2 * k;
+        t.tip[k] = reinterpret_cast<uint64_t>(I.states) + (kind == CHILD_TIP ? (size_t)id * I.Ppad : 0);
+        t.v[k] = kind == CHILD_SLOT ? id * nv : kNoSlot;
+        t.sc[k] = kind == CHILD_SLOT ? id * nc : kNoSlot;
+    }
+    t.dst = op.dad_slot * nv;
+    t.dsc = op.dad_slot * nc;
+    t.root = root;
+    tops[o] = t;
+    if (o == nops - 1)
+        for (int a = 1; a <= kTileAhead; a++) tops[o + a] = t;
+}
+
 // ---------------------------------------------------------------------------
 // computePartialInfo (tree/phylokernelnew.h:1008-1109): per op and child, the
 // eigen-basis transition rows echild[c][x][i] = evec[x][i] exp(eval[i] r_c t)
 // for an internal child, or the tip table leaf[s][c][x] =
 // sum_i echild[c][x][i] tip[s][i] (leaf[SU] = 1) for a tip child.
 // One workgroup per (op, child, category); tables are written in storage
-// precision.
+// precision. 4 states: also the steps' addresses (tops).
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
 k_prep_ops(const plk_op* __restrict__ ops, int nops, ModelDev m, int n, int C, int SU,
-           int table_size, T* __restrict__ tables) {
+           int table_size, T* __restrict__ tables, InstDev I, TileOp* __restrict__ tops) {
     // one block per (op, child, category); LDS: ex[n], then for a tip child
     // U[n][n] and the tip vectors [SU][n]
     extern __shared__ double sh[];
     const int o = blockIdx.x >> 1, k = blockIdx.x & 1, c = blockIdx.y;
     if (o >= nops) return;
+    if (tops && k == 0 && c == 0 && threadIdx.x == 0) make_tile_op<T>(I, ops, o, nops, tops);
     const plk_child ch = ops[o].child[k];
     double* ex = sh;
     for (int i = threadIdx.x; i < n; i += blockDim.x) ex[i] = exp(m.eval[i] * (m.rates[c] * ch.length));
     T* out = tables + (size_t)(2 * o + k) * table_size;
-    if (!ch.is_tip) {
+    if (!ch.is_tip || (n == 4 && sizeof(T) == 8)) {
         __syncthreads();
         if (n == kProtN) {
             // the matrix-core tile's fragment order
@@ -154,6 +283,14 @@ k_prep_ops(const plk_op* __restrict__ ops, int nops, ModelDev m, int n, int C, i
                 int x, i;
                 prot_frag_index(t, x, i);
                 oc[t] = x < 0 ? (T)0 : (T)(m.evec[x * n + i] * ex[i]);
+            }
+            return;
+        }
+        if (n == 4 && sizeof(T) == 8) {
+            T* step = tables + (size_t)2 * o * table_size;
+            for (int t = threadIdx.x; t < 16; t += blockDim.x) {
+                const T v = (T)(m.evec[t] * ex[t % 4]);
+                dna_frag(C, c, t / 4, t % 4, k, [&](int at) { step[at] = v; });
             }
             return;
         }
@@ -375,26 +512,24 @@ template <typename T, int N, int C>
 __device__ inline void op_load(const InstDev& I, int l_tip, int l_id, int r_tip, int r_id, int p, int c,
                                OpIn<T, N>& in) {
     using ST = typename Prec<T>::scale_t;
-    constexpr int block = N * C;
     const T* partial = reinterpret_cast<const T*>(I.partial);
     const ST* scale = reinterpret_cast<const ST*>(I.scale);
-    const size_t sidx = I.safe ? (size_t)p * C + c : (size_t)p;
     in.scl = in.scr = 0;
     if (l_tip) {
         in.sl = I.states[(size_t)l_id * I.Ppad + p];
     } else {
-        const T* src = partial + (size_t)l_id * I.slot_stride + (size_t)p * block + c * N;
+        const T* src = partial + Part<T, N, C>::at(I, l_id, p, c);
 #pragma unroll
-        for (int i = 0; i < N; i++) in.l[i] = src[i];
-        in.scl = scale[(size_t)l_id * I.scale_stride + sidx];
+        for (int i = 0; i < N; i++) in.l[i] = src[i * Part<T, N, C>::stride];
+        in.scl = scale[Part<T, N, C>::count_at(I, l_id, p, c)];
     }
     if (r_tip) {
         in.sr = I.states[(size_t)r_id * I.Ppad + p];
     } else {
-        const T* src = partial + (size_t)r_id * I.slot_stride + (size_t)p * block + c * N;
+        const T* src = partial + Part<T, N, C>::at(I, r_id, p, c);
 #pragma unroll
-        for (int i = 0; i < N; i++) in.r[i] = src[i];
-        in.scr = scale[(size_t)r_id * I.scale_stride + sidx];
+        for (int i = 0; i < N; i++) in.r[i] = src[i * Part<T, N, C>::stride];
+        in.scr = scale[Part<T, N, C>::count_at(I, r_id, p, c)];
     }
 }
 
@@ -402,12 +537,10 @@ template <typename T, int N, int C>
 __device__ inline void op_finish(const InstDev& I, const T* inv_sh, const T* tL, const T* tR, int l_tip,
                                  int r_tip, int dad_slot, int p, int c, const OpIn<T, N>& in) {
     using ST = typename Prec<T>::scale_t;
-    constexpr int block = N * C;
     T* partial = reinterpret_cast<T*>(I.partial);
     ST* scale = reinterpret_cast<ST*>(I.scale);
     const bool safe = I.safe != 0;
     T tmp[N];
-    const size_t sidx = safe ? (size_t)p * C + c : (size_t)p;
     if (l_tip) {
         const T* lut = tL + (in.sl * C + c) * N;
 #pragma unroll
@@ -458,10 +591,10 @@ __device__ inline void op_finish(const InstDev& I, const T* inv_sh, const T* tL,
             sc += k;
         }
     }
-    T* dst = partial + (size_t)dad_slot * I.slot_stride + (size_t)p * block + c * N;
+    T* dst = partial + Part<T, N, C>::at(I, dad_slot, p, c);
 #pragma unroll
-    for (int i = 0; i < N; i++) dst[i] = dadv[i];
-    if (safe || c == 0) scale[(size_t)dad_slot * I.scale_stride + sidx] = (ST)sc;
+    for (int i = 0; i < N; i++) dst[i * Part<T, N, C>::stride] = dadv[i];
+    if (Part<T, N, C>::counts(I, c)) scale[Part<T, N, C>::count_at(I, dad_slot, p, c)] = (ST)sc;
 }
 
 template <typename T, int N, int C>
@@ -473,6 +606,417 @@ __device__ inline void op_apply(const InstDev& I, const T* inv_sh, const T* tL, 
     op_finish<T, N, C>(I, inv_sh, tL, tR, l_tip, r_tip, dad_slot, p, c, in);
 }
 
+// ---------------------------------------------------------------------------
+// A whole op list for a wavefront's 64 (pattern, category) pairs, 4 states,
+// on the matrix cores. The same sums in the same order as op_finish: the 4x4
+// products are exact chains of fused multiply-adds.
+//
+// What bounds a step: with tables and children read through LDS and memory, a
+// step of a small tree took 2.0 us (two barriers, the tables' trip to LDS, the
+// dad's values back from L2), and its matrix rows took 384 bytes of LDS reads
+// a thread. A 4x4x4 product of four blocks takes one matrix element a lane
+// instead, its result is laid out as its operand, and so are the slots (Part):
+// a step is the children's products, their elementwise product and U^-1. No
+// barrier, no shuffle; a tip's vectors come from LDS, where they stay. A large
+// tree is bound by the vector memory path of its CU (16 bytes of a lane a
+// cycle and quad), so
+//   - the last two dads' values and counters stay in registers. In post-order
+//     every step but a cherry has the last one as a child: of a random tree's
+//     child reads a fifth remains;
+//   - what a step reads is loaded two steps ahead. Loads and stores share one
+//     in-order counter, so a wait for a load is one for all before it, but not
+//     for the stores of the two steps since;
+//   - a step makes few accesses: both children's matrices in one, and the tips'
+//     states through the scalar cache. Of 200 taxa x 100,000 sites' 858 us with
+//     13 vector accesses a step, 430 went into the stores, at the rate of a
+//     fill, 165 into children (most of them not needed, read past the end of
+//     a buffer), 110 into states and 108 into matrices, one after the other.
+// Measured, whole kernel, 198 steps: 1,000 patterns 415 -> 125 us, 99,390
+// patterns 1,153 -> 711 us in double (5.1 GB algorithmic, 2.6 GB written).
+typedef unsigned tile_u4 __attribute__((ext_vector_type(4)));
+using Buffer = __amdgpu_buffer_rsrc_t;
+
+// `bytes` from `base` on; reads past them give 0
+__device__ inline Buffer buffer_of(uint64_t base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
+}
+
+// the constant address space: a scalar load, whatever was stored before
+__device__ inline tile_u4 load_u4(uint64_t p) { return *(const __attribute__((address_space(4))) tile_u4*)p; }
+
+// The pairs of a wavefront, in the order of Part: pair j + 4b + 16g is lane
+// j + 4b + 16g's own (its state, its counter). The four pairs of a (b, g)
+// share a category, as a block of the matrix products does.
+template <int C>
+struct Pairs {
+    static constexpr int kPatterns = 64 / C;
+    __device__ static int cat(int b, int g) { return C == 1 ? 0 : C == 2 ? b & 1 : C == 4 ? b : b + 4 * (g & 1); }
+    __device__ static int cat(int lane) { return cat(lane >> 2 & 3, lane >> 4); }
+    __device__ static int pattern(int lane) {
+        const int j = lane & 3, b = lane >> 2 & 3, g = lane >> 4;
+        return C == 1 ? lane : C == 2 ? j + 4 * (b >> 1) + 8 * g : C == 4 ? j + 4 * g : j + 4 * (g >> 1);
+    }
+    // the pairs of pair 0's pattern; those of pair l's: kMask << (l & ~kBits)
+    static constexpr unsigned long long kMask = C == 1 ? 0x1ull : C == 2 ? 0x11ull : C == 4 ? 0x1111ull : 0x11111111ull;
+    static constexpr int kBits = 4 * (C - 1);
+};
+
+// 4x4 matrices times a wavefront's 4-vectors, four registers a lane:
+//   double  v_mfma_f64_4x4x4: four blocks of 4x4 by 4x4. A[i][k] of block b in
+//           lane i + 4b + 16k; B and D alike, D[i][j] in lane j + 4b + 16i. So
+//           register g of lane j + 4b + 16x holds value x of pair j + 4b + 16g
+//   float   v_mfma_f32_4x4x1: sixteen blocks, four steps of k. Register x of
+//           lane l holds value x of pair l
+template <typename T, int C> struct Mat4;
+template <int C> struct Mat4<double, C> {
+    static constexpr int kA = C == 8 ? 2 : 1;   // matrices of the even and odd registers
+    struct A {
+        double v[kA];
+    };
+    // both children's elements of a step (dna_frag); the same matrix M in every block
+    __device__ static void load(const Hbm<double>* step, int, int lane, A (&e)[2]) {
+        typedef double d2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int h = 0; h < kA; h++) {
+            const d2 w = ((const Hbm<d2>*)step)[64 * h + lane];
+            e[0].v[h] = w[0];
+            e[1].v[h] = w[1];
+        }
+    }
+    __device__ static A load_same(const double* M, int lane) {
+        A a;
+#pragma unroll
+        for (int h = 0; h < kA; h++) a.v[h] = M[(lane & 3) * 4 + (lane >> 4)];
+        return a;
+    }
+    __device__ static void mul(const A& a, const double (&b)[4], double (&d)[4]) {
+#pragma unroll
+        for (int g = 0; g < 4; g++) d[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.v[g % kA], b[g], 0.0, 0, 0, 0);
+    }
+    static constexpr int kRow = 1;              // a tip's row of its lookup: none, its vectors wait in LDS
+    // the states of a wavefront's patterns, in scalar registers where a
+    // register's pairs have theirs in one word of them (a vector load of single
+    // bytes takes the memory path as long as one of a kilobyte)
+    static constexpr bool kWords = C >= 4;
+    static constexpr int kStates = kWords ? 16 / C : 1;
+    __device__ static void load_slot(Buffer r, uint32_t at, double (&v)[4]) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const tile_u4 w = __builtin_amdgcn_raw_buffer_load_b128(r, at + 1024 * h, 0, 0);
+#pragma unroll
+            for (int m = 0; m < 2; m++)
+                v[2 * h + m] = __longlong_as_double((long long)((unsigned long long)w[2 * m + 1] << 32 | w[2 * m]));
+        }
+    }
+    __device__ static void store_slot(Buffer r, uint32_t at, const double (&d)[4]) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            tile_u4 w;
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                const unsigned long long u = (unsigned long long)__double_as_longlong(d[2 * h + m]);
+                w[2 * m] = (unsigned)u;
+                w[2 * m + 1] = (unsigned)(u >> 32);
+            }
+            __builtin_amdgcn_raw_buffer_store_b128(w, r, at + 1024 * h, 0, 0);
+        }
+    }
+    __device__ static void load_row(const Hbm<double>*, bool, int, int, double (&)[kRow]) {}
+    // a tip's product: its matrices times the tip vectors (the root leaf's: times 1, 0, 0, 0)
+    __device__ static void tip(const A& a, const double (&)[kRow], const unsigned (&st)[kStates], bool root,
+                               const double* tip_sh, int lane, double (&f)[4]) {
+        int s[4];
+        if constexpr (kWords) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) s[g] = st[C == 4 ? g : g >> 1] >> 8 * (lane & 3) & 0xff;
+        } else {
+            // row g of lanes holds the states of register g's pairs: each to every row
+            const auto w = __builtin_amdgcn_permlane32_swap(st[0], st[0], false, false);
+            const auto lo = __builtin_amdgcn_permlane16_swap(w[0], w[0], false, false);
+            const auto hi = __builtin_amdgcn_permlane16_swap(w[1], w[1], false, false);
+            s[0] = lo[0];
+            s[1] = lo[1];
+            s[2] = hi[0];
+            s[3] = hi[1];
+        }
+        double b[4];
+        if (root) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) b[g] = lane < 16 ? 1.0 : 0.0;
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; g++) b[g] = tip_sh[s[g] * 4 + (lane >> 4)];
+        }
+        mul(a, b, f);
+    }
+    // pairs with every value below the threshold, as a mask
+    __device__ static unsigned long long small(const double (&d)[4]) {
+        unsigned long long m[4], any = 0;
+#pragma unroll
+        for (int g = 0; g < 4; g++) any |= m[g] = __builtin_amdgcn_ballot_w64(fabs(d[g]) < Prec<double>::threshold);
+        if (!any) return 0;
+        unsigned long long out = 0;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            m[g] &= m[g] >> 32;
+            m[g] &= m[g] >> 16;
+            out |= (m[g] & 0xffff) << 16 * g;
+        }
+        return out;
+    }
+    // rescale the pairs for which `mine` holds; what their counters gain
+    template <bool>
+    __device__ static int rescale(double (&d)[4], bool mine, int lane) {
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(mine);
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            if (m >> (16 * g + (lane & 15)) & 1) d[g] = Prec<double>::apply(d[g], 1);
+        return mine ? 1 : 0;
+    }
+};
+template <int C> struct Mat4<float, C> {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    struct A {
+        float v[4];
+    };
+    // rows of both children's E[c][x][i]
+    __device__ static void load(const Hbm<float>* step, int table_size, int lane, A (&e)[2]) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const f4 w = *(const Hbm<f4>*)(step + c * table_size + Pairs<C>::cat(lane) * 16 + (lane & 3) * 4);
+#pragma unroll
+            for (int k = 0; k < 4; k++) e[c].v[k] = w[k];
+        }
+    }
+    __device__ static A load_same(const double* M, int lane) {
+        A a;
+#pragma unroll
+        for (int k = 0; k < 4; k++) a.v[k] = (float)M[(lane & 3) * 4 + k];
+        return a;
+    }
+    __device__ static void mul(const A& a, const float (&b)[4], float (&d)[4]) {
+        f4 acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(a.v[k], b[k], acc, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; r++) d[r] = acc[r];
+    }
+    static constexpr int kRow = 4;
+    static constexpr bool kWords = false;
+    static constexpr int kStates = 1;
+    __device__ static void load_slot(Buffer r, uint32_t at, float (&v)[4]) {
+        const tile_u4 w = __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0);
+#pragma unroll
+        for (int x = 0; x < 4; x++) v[x] = __uint_as_float(w[x]);
+    }
+    __device__ static void store_slot(Buffer r, uint32_t at, const float (&d)[4]) {
+        tile_u4 w;
+#pragma unroll
+        for (int x = 0; x < 4; x++) w[x] = __float_as_uint(d[x]);
+        __builtin_amdgcn_raw_buffer_store_b128(w, r, at, 0, 0);
+    }
+    // a tip's row of its lookup [SU+1][C][4] (others: the first)
+    __device__ static void load_row(const Hbm<float>* table, bool tip, int st, int lane, float (&row)[kRow]) {
+        const f4 w = *(const Hbm<f4>*)(table + (tip ? (st * C + Pairs<C>::cat(lane)) * 4 : 0));
+#pragma unroll
+        for (int x = 0; x < 4; x++) row[x] = w[x];
+    }
+    __device__ static void tip(const A&, const float (&row)[kRow], const unsigned (&)[kStates], bool, const double*, int,
+                               float (&f)[4]) {
+#pragma unroll
+        for (int x = 0; x < 4; x++) f[x] = row[x];
+    }
+    __device__ static float top(const float (&d)[4]) {
+        return fmax(fmax(fabs(d[0]), fabs(d[1])), fmax(fabs(d[2]), fabs(d[3])));
+    }
+    __device__ static unsigned long long small(const float (&d)[4]) {
+        return __builtin_amdgcn_ballot_w64(top(d) < Prec<float>::threshold);
+    }
+    // by the power of two that brings the pattern's (safe: the pair's) maximum into [0.5, 1)
+    template <bool kSafe>
+    __device__ static int rescale(float (&d)[4], bool mine, int lane) {
+        float m = top(d);
+        if (!kSafe)
+#pragma unroll
+            for (int w = 4; w < 4 * C; w <<= 1) m = fmax(m, __shfl_xor(m, w));
+        if (!mine || !Prec<float>::underflow(m)) return 0;
+        const int k = Prec<float>::exponent(m);
+#pragma unroll
+        for (int x = 0; x < 4; x++) d[x] = Prec<float>::apply(d[x], k);
+        return k;
+    }
+};
+
+// LDS of dna_ops: the tip vectors
+__host__ __device__ inline size_t dna_ops_smem(int SU) { return (size_t)(SU + 1) * 4 * sizeof(double); }
+
+// p_first: the workgroup's first of 256 / C patterns (uniform). tip_sh:
+// dna_ops_smem(SU). kFar: instances of dna_far, a buffer of its own for each slot.
+template <typename T, int C, bool kFar>
+__device__ inline void dna_ops(const InstDev& I, const ModelDev& m, const TileOp* tops, int nops, const T* tables_g,
+                               int table_size, int p_first, double* tip_sh) {
+    using ST = typename Prec<T>::scale_t;
+    using M = Mat4<T, C>;
+    using Pr = Pairs<C>;
+    if (nops == 0) return;
+    if (sizeof(T) == 8) {
+        for (int t = threadIdx.x; t < (I.SU + 1) * 4; t += kThreads) tip_sh[t] = m.tip[t];
+        __syncthreads();
+    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int p0 = p_first + wave * Pr::kPatterns;   // of the wavefront
+    const int q = Pr::pattern(lane);
+    const bool no_invar = I.invar[p0 + q] == 0.0;
+    const typename M::A inv = M::load_same(m.inv_evec, lane);
+    // the chunk's values and counters, and this lane's places in a slot of them
+    const size_t chunk = (size_t)(p0 / Pr::kPatterns) * I.chunk_slots;
+    constexpr uint32_t nv = kChunkValues<T>, nc = kChunkCounts<T>;
+    const uint64_t vbase = (uint64_t)I.partial + chunk * nv, cbase = (uint64_t)I.scale + chunk * nc;
+    const Buffer values_all = buffer_of(vbase, I.chunk_slots * nv), counts_all = buffer_of(cbase, I.chunk_slots * nc);
+    // the buffer that holds a slot, and where in it the slot begins
+    auto part = [](Buffer all, uint64_t base, uint32_t slot, uint32_t bytes) {
+        return kFar ? buffer_of(base + (uint64_t)slot * bytes, slot == kNoSlot ? 0 : bytes) : all;
+    };
+    auto from = [](uint32_t slot) { return kFar ? 0u : slot; };
+    const uint32_t vat = lane * 16, sat = lane * sizeof(ST);
+
+    struct Kids {
+        T v[2][4];                       // a slot's values
+        T row[2][M::kRow];               // float: a tip's row of its lookup
+        typename M::A e[2];              // the children's matrices
+        int sc[2];                       // the pair's counters
+    };
+    struct States {
+        unsigned w[2][M::kStates];
+    };
+    struct Desc {
+        tile_u4 end;                     // dst, dsc, kind, root of the step itself
+        tile_u4 tips, kids, kids_end;    // the step after next's
+    };
+    // float storage looks up a tip's row two steps ahead: its states come four ahead
+    constexpr bool kTipsAhead = M::kRow > 1;
+    const uint64_t tp = (uint64_t)tops;
+    auto desc = [&](int o) {
+        const uint64_t at = tp + (uint64_t)o * sizeof(TileOp);
+        return Desc{load_u4(at + 32), load_u4(at + 128), load_u4(at + 144), load_u4(at + 160)};
+    };
+    auto load_states = [&](const tile_u4 tips, unsigned kind, States& st) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const uint64_t row = ((uint64_t)tips[2 * k + 1] << 32 | tips[2 * k]) + p0;
+            if constexpr (M::kWords) {
+                // of another child: taxon 0's, not used
+                const auto* w = (const __attribute__((address_space(4))) unsigned*)row;
+#pragma unroll
+                for (int i = 0; i < M::kStates; i++) st.w[k][i] = w[i];
+            } else if ((kind >> 2 * k & 3) == CHILD_TIP) {
+                st.w[k][0] = ((const Hbm<uint8_t>*)row)[q];
+            }
+        }
+    };
+    const Hbm<T>* tab = (const Hbm<T>*)tables_g;
+    auto load_tables = [&](unsigned kind, const States& st, Kids& in) {
+        M::load(tab, table_size, lane, in.e);
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            M::load_row(tab + k * table_size, (kind >> 2 * k & 3) == CHILD_TIP, st.w[k][0], lane, in.row[k]);
+        tab += 2 * table_size;
+    };
+    // past the end of the buffers (kNoSlot) for a child that is no slot
+    auto load_slot = [&](const tile_u4 kids, int k, Kids& in) {
+        M::load_slot(part(values_all, vbase, kids[k], nv), vat + from(kids[k]), in.v[k]);
+        const Buffer counts = part(counts_all, cbase, kids[2 + k], nc);
+        const uint32_t at = sat + from(kids[2 + k]);
+        if (sizeof(ST) == 2) in.sc[k] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(counts, at, 0, 0);
+        else in.sc[k] = (int)__builtin_amdgcn_raw_buffer_load_b32(counts, at, 0, 0);
+    };
+
+    // even and odd steps have their own registers, since a copy would wait for
+    // the loads. Steps past the end repeat the last one's TileOp (kTileAhead),
+    // and read the tables of two steps more
+    Desc d_even, d_odd;
+    Kids even, odd;
+    States st_even, st_odd;                // of the step; float: of the step after next
+    T dad_even[4] = {}, dad_odd[4] = {};   // the last two dads
+    int sc_even = 0, sc_odd = 0;
+    {
+        const tile_u4 k0 = load_u4(tp + 16), k1 = load_u4(tp + sizeof(TileOp) + 16);
+        const tile_u4 e0 = load_u4(tp + 32), e1 = load_u4(tp + sizeof(TileOp) + 32);
+        load_states(load_u4(tp), e0[2], st_even);
+        load_states(load_u4(tp + sizeof(TileOp)), e1[2], st_odd);
+        // slots last and unconditionally: the loop's first waits must not be
+        // shorter than its later ones, which have stores to look past
+        load_tables(e0[2], st_even, even);
+        load_tables(e1[2], st_odd, odd);
+        for (int k = 0; k < 2; k++) load_slot(k0, k, even);
+        for (int k = 0; k < 2; k++) load_slot(k1, k, odd);
+        d_even = desc(0);
+        d_odd = desc(1);
+        if constexpr (kTipsAhead) {
+            load_states(d_even.tips, CHILD_TIP | CHILD_TIP << 2, st_even);
+            load_states(d_odd.tips, CHILD_TIP | CHILD_TIP << 2, st_odd);
+            d_even.tips = load_u4(tp + 4 * sizeof(TileOp));
+            d_odd.tips = load_u4(tp + 5 * sizeof(TileOp));
+        }
+    }
+    auto step = [&](int o, Desc& d, Kids& in, States& st, T(&dad)[4], int& dad_sc, const T(&last)[4], int last_sc) {
+        T f[2][4];
+        int sc = 0;
+        const unsigned kinds = d.end[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const unsigned kind = kinds >> 2 * k & 3;
+            if (kind == CHILD_TIP) {
+                M::tip(in.e[k], in.row[k], st.w[k], d.end[3] >> k & 1, tip_sh, lane, f[k]);
+            } else if (kind == CHILD_LAST) {
+                M::mul(in.e[k], last, f[k]);
+                sc += last_sc;
+            } else if (kind == CHILD_LAST2) {
+                M::mul(in.e[k], dad, f[k]);
+                sc += dad_sc;
+            } else {
+                M::mul(in.e[k], in.v[k], f[k]);
+                sc += in.sc[k];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) f[0][i] *= f[1][i];
+        M::mul(inv, f[0], dad);
+        // a pattern is rescaled when all its categories (safe mode: the pair)
+        // are below the threshold; tip-tip steps never
+        const unsigned long long small = M::small(dad);
+        if (small && kinds != (CHILD_TIP | CHILD_TIP << 2)) {
+            int l = lane;
+            asm("" : "+v"(l));   // masks of the lane are made here, not kept through the list
+            if (I.safe) sc += M::template rescale<true>(dad, (small >> l & 1) && no_invar, l);
+            else sc += M::template rescale<false>(
+                dad, (small >> (l & ~Pr::kBits) & Pr::kMask) == Pr::kMask && no_invar, l);
+        }
+        dad_sc = sc;
+        // the step after next's loads, then this step's stores: a wait for the
+        // loads is then not one for these stores (a child that is a slot was
+        // stored two steps ago or earlier)
+        load_tables(d.kids_end[2], st, in);
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            if ((d.kids_end[2] >> 2 * k & 3) == CHILD_SLOT) load_slot(d.kids, k, in);
+        load_states(d.tips, kTipsAhead ? CHILD_TIP | CHILD_TIP << 2 : d.kids_end[2], st);
+        M::store_slot(part(values_all, vbase, d.end[0], nv), vat + from(d.end[0]), dad);
+        const Buffer counts = part(counts_all, cbase, d.end[1], nc);
+        const uint32_t at = sat + from(d.end[1]);
+        if (sizeof(ST) == 2) __builtin_amdgcn_raw_buffer_store_b16((unsigned short)sc, counts, at, 0, 0);
+        else __builtin_amdgcn_raw_buffer_store_b32(sc, counts, at, 0, 0);
+        d = desc(o + 2);
+        if constexpr (kTipsAhead) d.tips = load_u4(tp + (uint64_t)(o + 6) * sizeof(TileOp));
+    };
+    int o = 0;
+    for (; o + 1 < nops; o += 2) {
+        step(o, d_even, even, st_even, dad_even, sc_even, dad_odd, sc_odd);
+        step(o + 1, d_odd, odd, st_odd, dad_odd, sc_odd, dad_even, sc_even);
+    }
+    if (o < nops) step(o, d_even, even, st_even, dad_even, sc_even, dad_odd, sc_odd);
+}
+
 // Branch ends for (p, c): node partial nv, dad partial (or tip vector from
 // tip_sh) dv, the summed scale counter and, in safe mode, the per-category
 // adjustment relative to the least-scaled category.
@@ -481,15 +1025,13 @@ __device__ inline void load_branch(const InstDev& I, plk_end node, plk_end dad, 
                                    int p, int c, double* nv, double* dv, int& minsc,
                                    double& adjust) {
     using ST = typename Prec<T>::scale_t;
-    constexpr int block = N * C;
     const T* partial = reinterpret_cast<const T*>(I.partial);
     const ST* scale = reinterpret_cast<const ST*>(I.scale);
     const bool safe = I.safe != 0;
-    const size_t sidx = safe ? (size_t)p * C + c : (size_t)p;
-    const T* nsrc = partial + (size_t)node.id * I.slot_stride + (size_t)p * block + c * N;
+    const T* nsrc = partial + Part<T, N, C>::at(I, node.id, p, c);
 #pragma unroll
-    for (int i = 0; i < N; i++) nv[i] = (double)nsrc[i];
-    int sc = scale[(size_t)node.id * I.scale_stride + sidx];
+    for (int i = 0; i < N; i++) nv[i] = (double)nsrc[i * Part<T, N, C>::stride];
+    int sc = scale[Part<T, N, C>::count_at(I, node.id, p, c)];
     if (dad.is_tip) {
         if (tip_sh) {   // callers that use a val-weighted lookup pass nullptr
             const int s = I.states[(size_t)dad.id * I.Ppad + p];
@@ -498,10 +1040,10 @@ __device__ inline void load_branch(const InstDev& I, plk_end node, plk_end dad, 
             for (int i = 0; i < N; i++) dv[i] = tp[i];
         }
     } else {
-        const T* dsrc = partial + (size_t)dad.id * I.slot_stride + (size_t)p * block + c * N;
+        const T* dsrc = partial + Part<T, N, C>::at(I, dad.id, p, c);
 #pragma unroll
-        for (int i = 0; i < N; i++) dv[i] = (double)dsrc[i];
-        sc += scale[(size_t)dad.id * I.scale_stride + sidx];
+        for (int i = 0; i < N; i++) dv[i] = (double)dsrc[i * Part<T, N, C>::stride];
+        sc += scale[Part<T, N, C>::count_at(I, dad.id, p, c)];
     }
     minsc = sc;
     adjust = 1.0;
@@ -528,46 +1070,27 @@ __device__ inline void theta_apply(const InstDev& I, plk_end node, plk_end dad, 
 // Fused post-order traversal over the op list followed, per mode, by the
 // branch lnL (computeLikelihoodBranchSIMD 2753-3104) or the theta buffer of
 // the branch (node, dad).
-template <typename T, int N, int C>
-__global__ void __launch_bounds__(kThreads)
-k_traverse(InstDev I, ModelDev m, const plk_op* __restrict__ ops, int nops,
+template <typename T, int N, int C, bool kFar>
+__global__ void __launch_bounds__(kThreads, 4)
+k_traverse(InstDev I, ModelDev m, const TileOp* __restrict__ tops, int nops,
            const T* __restrict__ tables, int table_size, int mode, plk_end node, plk_end dad,
            const double* __restrict__ root_tab, double* __restrict__ block_sums) {
     extern __shared__ __align__(16) unsigned char smem[];
-    T* inv_sh = reinterpret_cast<T*>(smem);                 // [N*N]
-    T* tab_sh = inv_sh + N * N;                              // [2][table_size]
     constexpr int PB = kThreads / C;
     constexpr int block = N * C;
     const int c = threadIdx.x % C;
     const int p = blockIdx.x * PB + threadIdx.x / C;
-    const bool live = p < I.Ppad;
+    const bool live = p < I.Ppad;                            // every thread: PB divides Ppad
 
-    for (int t = threadIdx.x; t < N * N; t += kThreads) inv_sh[t] = (T)m.inv_evec[t];
-
-    for (int o = 0; o < nops; o++) {
-        const plk_op op = ops[o];
-        int left = 0, right = 1;
-        if (!op.child[0].is_tip && op.child[1].is_tip) { left = 1; right = 0; }
-        const plk_child L = op.child[left], R = op.child[right];
-        const int szL = L.is_tip ? (I.SU + 1) * block : block * N;
-        const int szR = R.is_tip ? (I.SU + 1) * block : block * N;
-        __syncthreads();
-        const T* gL = tables + (size_t)(2 * o + left) * table_size;
-        const T* gR = tables + (size_t)(2 * o + right) * table_size;
-        for (int t = threadIdx.x; t < szL; t += kThreads) tab_sh[t] = gL[t];
-        for (int t = threadIdx.x; t < szR; t += kThreads) tab_sh[table_size + t] = gR[t];
-        __syncthreads();
-        if (live)
-            op_apply<T, N, C>(I, inv_sh, tab_sh, tab_sh + table_size, L.is_tip, L.id, R.is_tip, R.id,
-                              op.dad_slot, p, c);
-    }
+    static_assert(N == 4, "20 and 61 states have their own traversal kernels");
+    dna_ops<T, C, kFar>(I, m, tops, nops, tables, table_size, blockIdx.x * PB, reinterpret_cast<double*>(smem));
 
     if (mode == MODE_PARTIALS) return;
 
     // ---- root stage ---------------------------------------------------------
     // MODE_BRANCH: root_tab = val[c][i] then, for a tip dad, lut[s][c][i] = val * tip
     // MODE_THETA:  the eigen-basis tip vectors
-    double* root_sh = reinterpret_cast<double*>(tab_sh);
+    double* root_sh = reinterpret_cast<double*>(smem);
     __syncthreads();
     if (mode == MODE_BRANCH) {
         const int root_size = block + (dad.is_tip ? (I.SU + 1) * block : 0);

@@ -63,10 +63,14 @@ __device__ inline void nr_trans_block(const NrDev& D, int m, double len, double*
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
 k_nr_prep_ops(const plk_op* __restrict__ ops, const uint8_t* __restrict__ flags, int nops, NrDev D,
-              const double* __restrict__ tip, int SU, int table_size, T* __restrict__ tables) {
+              const double* __restrict__ tip, int SU, int table_size, T* __restrict__ tables, InstDev I,
+              TileOp* __restrict__ tops) {
     extern __shared__ double sh[];
     const int o = blockIdx.x >> 1, k = blockIdx.x & 1, c = blockIdx.y;
     if (o >= nops) return;
+    if (tops && k == 0 && c == 0 && threadIdx.x == 0)
+        make_tile_op<T>(I, ops, o, nops, tops,
+                        (flags[2 * o] & kNrRootLeaf ? 1 : 0) | (flags[2 * o + 1] & kNrRootLeaf ? 2 : 0));
     const int n = D.n, C = D.C, m = D.mix[c];
     const plk_child ch = ops[o].child[k];
     const int fl = flags[2 * o + k];
@@ -75,6 +79,16 @@ k_nr_prep_ops(const plk_op* __restrict__ ops, const uint8_t* __restrict__ flags,
     nr_trans_block(D, m, D.rate[c] * ch.length, ex, P);
     const bool tr = (fl & kNrTowardRoot) != 0;
     T* out = tables + (size_t)(2 * o + k) * table_size;
+    if (n == 4 && sizeof(T) == 8) {
+        // dna_ops multiplies the root leaf's matrix by 1, 0, 0, 0
+        T* step = tables + (size_t)2 * o * table_size;
+        for (int t = threadIdx.x; t < 16; t += blockDim.x) {
+            const int x = t / 4, i = t % 4;
+            const T v = fl & kNrRootLeaf ? (i == 0 ? (T)D.pi[(size_t)m * n + x] : (T)0) : (T)(tr ? P[i * n + x] : P[x * n + i]);
+            dna_frag(C, c, x, i, k, [&](int at) { step[at] = v; });
+        }
+        return;
+    }
     if (!ch.is_tip) {
         if (n == kProtN) {
             T* oc = out + (size_t)c * kProtFrag;
@@ -219,14 +233,14 @@ k_nr_root(InstDev I, NrRoot R, double* __restrict__ block_sums) {
     double u0 = 0.0, u1 = 0.0, u2 = 0.0;
     int a = 0, b = 0;
     if (live) {
-        const T* pn = reinterpret_cast<const T*>(I.partial) + R.node_slot * I.slot_stride + ((size_t)p * C + c) * N;
+        const T* pn = reinterpret_cast<const T*>(I.partial) + Part<T, N, C>::at(I, R.node_slot, p, c);
         if (R.dad_tip) {
             const int s = I.states[(size_t)R.dad_taxon * I.Ppad + p];
             const size_t ls = (size_t)(I.SU + 1) * C * N;
             const double* l0 = R.lut + ((size_t)s * C + c) * N;
 #pragma unroll
             for (int x = 0; x < N; x++) {
-                const double nv = (double)pn[x];
+                const double nv = (double)pn[x * Part<T, N, C>::stride];
                 u0 = fma(nv, l0[x], u0);
                 if (R.derv) {
                     u1 = fma(nv, l0[ls + x], u1);
@@ -234,10 +248,10 @@ k_nr_root(InstDev I, NrRoot R, double* __restrict__ block_sums) {
                 }
             }
         } else {
-            const T* pd = reinterpret_cast<const T*>(I.partial) + R.dad_slot * I.slot_stride + ((size_t)p * C + c) * N;
+            const T* pd = reinterpret_cast<const T*>(I.partial) + Part<T, N, C>::at(I, R.dad_slot, p, c);
             double dv[N];
 #pragma unroll
-            for (int y = 0; y < N; y++) dv[y] = (double)pd[y];
+            for (int y = 0; y < N; y++) dv[y] = (double)pd[y * Part<T, N, C>::stride];
             const double* T0 = R.T + (size_t)c * N * N;
             const double* T1 = T0 + (size_t)C * N * N;
             const double* T2 = T1 + (size_t)C * N * N;
@@ -251,15 +265,16 @@ k_nr_root(InstDev I, NrRoot R, double* __restrict__ block_sums) {
                         v2 = fma(T2[x * N + y], dv[y], v2);
                     }
                 }
-                const double nv = (double)pn[x];
+                const double nv = (double)pn[x * Part<T, N, C>::stride];
                 u0 = fma(nv, v0, u0);
                 u1 = fma(nv, v1, u1);
                 u2 = fma(nv, v2, u2);
             }
         }
         if (I.safe) {
-            a = reinterpret_cast<const S*>(I.scale)[R.node_slot * I.scale_stride + (size_t)p * C + c];
-            b = R.dad_tip ? 0 : (int)reinterpret_cast<const S*>(I.scale)[R.dad_slot * I.scale_stride + (size_t)p * C + c];
+            const S* sc = reinterpret_cast<const S*>(I.scale);
+            a = sc[Part<T, N, C>::count_at(I, R.node_slot, p, c)];
+            b = R.dad_tip ? 0 : (int)sc[Part<T, N, C>::count_at(I, R.dad_slot, p, c)];
         }
     }
     // every lane takes part in the shuffles
@@ -274,9 +289,9 @@ k_nr_root(InstDev I, NrRoot R, double* __restrict__ block_sums) {
     } else {
         minsc = 0;
         if (live) {
-            const S* sn = reinterpret_cast<const S*>(I.scale) + R.node_slot * I.scale_stride;
-            minsc = (int)sn[p];
-            if (!R.dad_tip) minsc += (int)reinterpret_cast<const S*>(I.scale)[R.dad_slot * I.scale_stride + p];
+            const S* sc = reinterpret_cast<const S*>(I.scale);
+            minsc = (int)sc[Part<T, N, C>::count_at(I, R.node_slot, p, c)];
+            if (!R.dad_tip) minsc += (int)sc[Part<T, N, C>::count_at(I, R.dad_slot, p, c)];
         }
         minsd = minsc;
     }

@@ -494,18 +494,17 @@ __device__ inline bool theta_first_eval(const SweepArgs& a, const SweepRes<T>& R
         const int tile = t0 + m * gridDim.x;
         if (tile >= ntiles) break;
         const int p = tile * PB + threadIdx.x / C;
-        const size_t sidx = I.safe ? (size_t)p * C + c : (size_t)p;
-        const T* nsrc = partial + (size_t)node.id * I.slot_stride + (size_t)p * block + c * N;
+        const T* nsrc = partial + Part<T, N, C>::at(I, node.id, p, c);
 #pragma unroll
-        for (int i = 0; i < N; i++) nr[m][i] = nsrc[i];
-        scr[m] = scale[(size_t)node.id * I.scale_stride + sidx];
+        for (int i = 0; i < N; i++) nr[m][i] = nsrc[i * Part<T, N, C>::stride];
+        scr[m] = scale[Part<T, N, C>::count_at(I, node.id, p, c)];
         if (dad.is_tip) {
             sr[m] = I.states[(size_t)dad.id * I.Ppad + p];
         } else {
-            const T* dsrc = partial + (size_t)dad.id * I.slot_stride + (size_t)p * block + c * N;
+            const T* dsrc = partial + Part<T, N, C>::at(I, dad.id, p, c);
 #pragma unroll
-            for (int i = 0; i < N; i++) dr[m][i] = dsrc[i];
-            scr[m] += scale[(size_t)dad.id * I.scale_stride + sidx];
+            for (int i = 0; i < N; i++) dr[m][i] = dsrc[i * Part<T, N, C>::stride];
+            scr[m] += scale[Part<T, N, C>::count_at(I, dad.id, p, c)];
         }
     }
 #pragma unroll
