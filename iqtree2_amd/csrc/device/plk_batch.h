@@ -20,7 +20,7 @@ struct BatchItem {
     ModelDev m;
     const plk_op* ops;     // this instance's ops inside the batch op array
     const void* tables;    // [nops][2][table_size] storage precision (4 states: and two steps more)
-    const TileOp* tops;    // 4 states: the ops as dna_ops reads them
+    const TileOp* tops;    // the ops as dna_ops and prot_ops read them
     const double* root;    // val[C][n] then, for a tip dad, lut[SU+1][C][n]
     int nops;
     int table_size;
@@ -48,6 +48,16 @@ __device__ inline void prep_child_table(const BatchItem& it, const plk_child ch,
             const int c = t / nn, r = t - c * nn;
             const T v = (T)(ev_sh[r] * ex[c * n + r % n]);
             dna_frag(C, c, r / n, r % n, k, [&](int at) { step[at] = v; });
+        }
+        return;
+    }
+    const bool prot = n == kProtN && sizeof(T) == 8;
+    if (prot && (!ch.is_tip || !prot_lut(SU))) {
+        for (int t = threadIdx.x; t < C * kProtBlocks; t += kThreads) {
+            const int c = t / kProtBlocks, r = t - c * kProtBlocks;
+            int x, i;
+            prot_block_index(r, x, i);
+            step[(2 * c + k) * kProtKid + r] = x < 0 ? (T)0 : (T)(ev_sh[x * n + i] * ex[c * n + i]);
         }
         return;
     }
@@ -81,7 +91,8 @@ __device__ inline void prep_child_table(const BatchItem& it, const plk_child ch,
             v = ev[0] * e[0] * tp[0];
             for (int i = 1; i < n; i++) v += ev[i] * e[i] * tp[i];
         }
-        out[t] = (T)v;
+        if (prot) step[(2 * c + k) * kProtKid + s * n + x] = (T)v;
+        else out[t] = (T)v;
     }
 }
 
@@ -117,7 +128,7 @@ k_prep_batch(const BatchItem* __restrict__ items, const double* __restrict__ len
             else
                 prep_child_table<double>(it, op.child[k], k, ev_sh, tp_sh, ex + k * nv, reinterpret_cast<double*>(tables) + off);
         }
-        if (n == 4 && threadIdx.x == 0) {
+        if ((n == 4 || (n == kProtN && !it.f32)) && threadIdx.x == 0) {
             TileOp* tops = hbm(const_cast<TileOp*>(it.tops));
             if (it.f32) make_tile_op<float>(it.I, it.ops, o, it.nops, tops);
             else make_tile_op<double>(it.I, it.ops, o, it.nops, tops);
@@ -152,14 +163,15 @@ __device__ inline double branch_end_stream(const InstDev& I, plk_end node, plk_e
     const ST* scale = reinterpret_cast<const ST*>(I.scale);
     const bool safe = I.safe != 0;
     const size_t sidx = safe ? (size_t)p * C + c : (size_t)p;
-    const T* nv = partial + (size_t)node.id * I.slot_stride + (size_t)p * block + c * N;
+    using L = Part<T, N, C>;
+    const T* nv = partial + L::at(I, node.id, p, c);
     int sc = scale[(size_t)node.id * I.scale_stride + sidx];
     const T* dv = nullptr;
     int s = 0;
     if (dad.is_tip) {
         s = I.states[(size_t)dad.id * I.Ppad + p];
     } else {
-        dv = partial + (size_t)dad.id * I.slot_stride + (size_t)p * block + c * N;
+        dv = partial + L::at(I, dad.id, p, c);
         sc += scale[(size_t)dad.id * I.scale_stride + sidx];
     }
     int minsc = sc;
@@ -173,10 +185,10 @@ __device__ inline double branch_end_stream(const InstDev& I, plk_end node, plk_e
         if (dad.is_tip) {
             const double* tp = tip_eig + s * N;
 #pragma unroll 4
-            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i] * tp[i] * adjust);
+            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i * L::stride] * tp[i] * adjust);
         } else {
 #pragma unroll 4
-            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i] * (double)dv[i] * adjust);
+            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i * L::stride] * (double)dv[i * L::stride] * adjust);
         }
         if (c == 0) I.buffer_scale[p] = (double)minsc * Prec<T>::log_unit;
         return 0.0;
@@ -186,12 +198,12 @@ __device__ inline double branch_end_stream(const InstDev& I, plk_end node, plk_e
         const double* lut = root_sh + block + (s * C + c) * N;
         lhc = lut[0] * (double)nv[0];
 #pragma unroll 1
-        for (int i = 1; i < N; i++) lhc = fma(lut[i], (double)nv[i], lhc);
+        for (int i = 1; i < N; i++) lhc = fma(lut[i], (double)nv[i * L::stride], lhc);
     } else {
         const double* val = root_sh + c * N;
         lhc = val[0] * (double)dv[0] * (double)nv[0];
 #pragma unroll 1
-        for (int i = 1; i < N; i++) lhc = fma(val[i] * (double)dv[i], (double)nv[i], lhc);
+        for (int i = 1; i < N; i++) lhc = fma(val[i] * (double)dv[i * L::stride], (double)nv[i * L::stride], lhc);
     }
     if (minsc_out) *minsc_out = minsc;
     return safe ? group_sum_sumvec<C>(lhc * adjust) : group_sum_ordered<C>(lhc);
@@ -201,15 +213,18 @@ __device__ inline double branch_end_stream(const InstDev& I, plk_end node, plk_e
 constexpr int kBatchSub = 4;
 
 // Dynamic LDS bytes batch_tile uses for one item shape: what its op list needs
-// (4 states: dna_ops; 20 states: the maxima of prot_ops_tile, 2 x kBatchSub x
-// C x 16), then the root tables.
+// (4 states: dna_ops; 20 states: prot_ops, or in float storage the maxima of
+// prot_ops_tile, 2 x kBatchSub x C x 16), then the root tables.
 __host__ __device__ inline size_t batch_smem_bytes(int n, int C, int SU, int table_size, size_t elem) {
     const size_t root = (size_t)(SU + 2) * n * C * 8;
     if (n == kCodonN) return (size_t)2 * n * kCodonStride * elem;   // E | U^-1; root rows stay in HBM
+    if (n == kProtN && elem == 8) {
+        const size_t ops = prot_ops_smem(SU, 4);
+        return ops > root ? ops : root;
+    }
     if (n == kProtN) {
         const size_t mf = (size_t)2 * kBatchSub * C * 16 * elem;
-        const size_t rt = (size_t)n * n * elem + root;
-        return mf > rt ? mf : rt;
+        return mf > root ? mf : root;
     }
     const size_t ops = dna_ops_smem(SU);
     return ops > root ? ops : root;
@@ -243,6 +258,11 @@ __device__ __forceinline__ double batch_tile(const BatchItem& it, int tile, unsi
         __syncthreads();
         for (int cc = 0; cc < C; cc++)
             codon_ops_tile<T>(I, ops, it.nops, tables, it.table_size, cc, tile * PB, e_m, inv_m);
+    } else if constexpr (N == 20 && sizeof(T) == 8) {
+        // a workgroup's 32 patterns twice
+        static_assert(PB == 2 * kProtPatterns, "two blocks a tile");
+        for (int h = 0; h < 2; h++)
+            prot_ops<C>(I, m, it.tops, it.nops, tables, it.table_size, tile * PB + h * kProtPatterns, smem);
     } else if constexpr (N == 20) {
         // protein: the matrix-core tile of the lone traversal kernel, every
         // wave one category of four 16-pattern sub-tiles
@@ -252,7 +272,7 @@ __device__ __forceinline__ double batch_tile(const BatchItem& it, int tile, unsi
     } else {
         dna_ops<T, C, false>(I, m, it.tops, it.nops, tables, it.table_size, tile * PB, reinterpret_cast<double*>(smem));
     }
-    double* root_sh = reinterpret_cast<double*>(smem) + (N == kProtN ? N * N * sizeof(T) / 8 : 0);
+    double* root_sh = reinterpret_cast<double*>(smem);
     const plk_end node = it.node, dad = it.dad;
     __syncthreads();
     if (it.mode == BATCH_THETA) {
@@ -317,7 +337,7 @@ __device__ __forceinline__ double batch_tile(const BatchItem& it, int tile, unsi
 // fused DNA + protein launch; codon tiles (63 KB of LDS) always run in a
 // launch of their own class, so they do not lower the others' occupancy.
 enum BatchClass {
-    BC_DNA64 = 1, BC_PROT64 = 2, BC_DNA32 = 4, BC_PROT32 = 8, BC_ALL = 15,
+    BC_DNA64 = 1, BC_PROT64 = 2, BC_DNA32 = 4, BC_PROT32 = 8, BC_ALL = 15, BC_F64 = 3, BC_F32 = 12,
     BC_COD64 = 16, BC_COD32 = 32
 };
 constexpr int kBatchClasses = 6;
@@ -343,12 +363,14 @@ struct XcdSplit {
 // is drained; every workgroup ends after trying each segment's counter. MASK
 // names the instance classes the launch may meet; a tile's code path is
 // uniform across its workgroup.
-// The protein classes are held to 3 (FP64, <= 168 registers) and 4 (FP32,
-// <= 128) waves per SIMD, which they fit without spilling; the compiler's
-// own choice left each one wave lower.
+// The classes with protein in FP64 are held to 3 waves per SIMD (168
+// registers), the others of DNA and protein to 4, without spills in their
+// loops; the compiler's own choice left each one wave or more lower. Classes
+// of one storage have a fused kernel of their own: 90 partitions in FP32,
+// DNA and protein, 737 us fused in four waves, 878 in two launches.
 template <int MASK>
 __global__ void __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(MASK == BC_PROT64 ? 3 : (MASK == BC_PROT32 || MASK == BC_DNA64 || MASK == BC_DNA32 ? 4 : 1))))
+__attribute__((amdgpu_waves_per_eu(MASK & ~BC_ALL ? 1 : MASK & BC_PROT64 ? 3 : 4)))
 k_batch(const BatchItem* __restrict__ items, const int* __restrict__ tile_item, XcdSplit xs,
         unsigned* __restrict__ counters, double* __restrict__ tile_sums) {
     extern __shared__ __align__(16) unsigned char smem[];

@@ -250,14 +250,15 @@ k_root_stream(InstDev I, ModelDev m, int mode, plk_end node, plk_end dad,
     const ST* scale = reinterpret_cast<const ST*>(I.scale);
     const bool safe = I.safe != 0;
     const size_t sidx = safe ? (size_t)p * C + c : (size_t)p;
-    const T* nv = partial + (size_t)node.id * I.slot_stride + (size_t)p * block + c * N;
+    using L = Part<T, N, C>;
+    const T* nv = partial + L::at(I, node.id, p, c);
     int sc = scale[(size_t)node.id * I.scale_stride + sidx];
     const T* dv = nullptr;
     int s = 0;
     if (dad.is_tip) {
         s = I.states[(size_t)dad.id * I.Ppad + p];
     } else {
-        dv = partial + (size_t)dad.id * I.slot_stride + (size_t)p * block + c * N;
+        dv = partial + L::at(I, dad.id, p, c);
         sc += scale[(size_t)dad.id * I.scale_stride + sidx];
     }
     // safe mode: per-category counters aligned to the least-scaled category
@@ -271,9 +272,9 @@ k_root_stream(InstDev I, ModelDev m, int mode, plk_end node, plk_end dad,
         T* th = reinterpret_cast<T*>(I.theta) + (size_t)p * block + c * N;
         if (dad.is_tip) {
             const double* tp = m.tip + s * N;
-            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i] * tp[i] * adjust);
+            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i * L::stride] * tp[i] * adjust);
         } else {
-            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i] * (double)dv[i] * adjust);
+            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i * L::stride] * (double)dv[i * L::stride] * adjust);
         }
         if (c == 0) I.buffer_scale[p] = (double)minsc * Prec<T>::log_unit;
         return;
@@ -282,11 +283,11 @@ k_root_stream(InstDev I, ModelDev m, int mode, plk_end node, plk_end dad,
     if (dad.is_tip) {
         const double* lut = root_tab + block + (size_t)(s * C + c) * N;
         lhc = lut[0] * (double)nv[0];
-        for (int i = 1; i < N; i++) lhc = fma(lut[i], (double)nv[i], lhc);
+        for (int i = 1; i < N; i++) lhc = fma(lut[i], (double)nv[i * L::stride], lhc);
     } else {
         const double* val = root_tab + c * N;
         lhc = val[0] * (double)dv[0] * (double)nv[0];
-        for (int i = 1; i < N; i++) lhc = fma(val[i] * (double)dv[i], (double)nv[i], lhc);
+        for (int i = 1; i < N; i++) lhc = fma(val[i] * (double)dv[i * L::stride], (double)nv[i * L::stride], lhc);
     }
     const double lh0 = safe ? group_sum_sumvec<C>(lhc * adjust) : group_sum_ordered<C>(lhc);
     double contrib = 0.0;

@@ -13,6 +13,7 @@
 #include <unordered_map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "plk.h"
@@ -125,7 +126,7 @@ struct Instance {
     unsigned char* sw_tabs = nullptr; // codon sweep: two steps' child tables
     size_t sw_tabs_cap = 0;
     void* tables = nullptr;
-    TileOp* tops = nullptr;           // 4 states: the staged ops as dna_ops reads them
+    TileOp* tops = nullptr;           // the staged ops as dna_ops and prot_ops read them
     bool patterns_set = false, model_set = false, theta_ready = false, ptn_lh_ready = false;
     double theta_length = 0.0;
     // Fitch parsimony state (allocated by the first parsimony call)
@@ -166,6 +167,11 @@ size_t alloc_class(size_t bytes);
 int stored_slots(const plk_instance_desc* d) { return d->nstates == 4 ? d->nslots | 1 : d->nslots; }
 int stored_counts(const plk_instance_desc* d) { return d->safe_numeric || d->nstates == 4 ? d->ncat : 1; }
 
+// op lists that the traversal reads as TileOps
+bool has_tile_ops(const plk_instance_desc* d) {
+    return d->nstates == 4 || (d->nstates == kProtN && d->precision != PLK_PREC_F32);
+}
+
 // red_out: 8 reduced scalars, then four values per unobserved pattern of
 // +ASC when there are at most kAscMax of them (the constant patterns of
 // ASC_VARIANT, one per state); the larger sets of ASC_INFORMATIVE live in
@@ -181,7 +187,9 @@ size_t footprint_of(const plk_instance_desc* d, int Ppad) {
     const size_t n = d->nstates, SU = d->state_unknown;
     const size_t block = n * d->ncat;
     const size_t ncnt = stored_counts(d);
-    const size_t table = n == 4 ? dna_table_size(d->ncat, d->state_unknown, elem) : std::max(block * n, (SU + 1) * block);
+    const size_t table = n == 4        ? dna_table_size(d->ncat, d->state_unknown, elem)
+                         : n == kProtN ? prot_table_size(d->ncat, d->state_unknown, elem)
+                                       : std::max(block * n, (SU + 1) * block);
     const size_t bufs[] = {
         (size_t)d->ntaxa * Ppad,                                  // states
         (size_t)Ppad * 8, (size_t)Ppad * 8,                       // freq, invar
@@ -195,7 +203,7 @@ size_t footprint_of(const plk_instance_desc* d, int Ppad) {
         (SU + 2) * block * 8,                                     // root tables
         sizeof(plk_op) * (size_t)d->nslots,                       // ops of a full traversal
         (size_t)(d->nslots + 2) * 2 * table * elem,               // and their tables
-        d->nstates == 4 ? sizeof(TileOp) * (size_t)(d->nslots + kTileAhead) : 0,
+        has_tile_ops(d) ? sizeof(TileOp) * (size_t)(d->nslots + kTileAhead) : 0,
     };
     size_t b = 0;
     for (size_t x : bufs)
@@ -276,7 +284,7 @@ struct plk_context {
     struct BatchTune {
         int next = 0;            // next candidate to time
         float best_ms = 1e30f;
-        int split = 1, bpc = 2;  // best so far (default until every candidate ran)
+        int split = 0, bpc = 4;  // best so far
         bool done = false;
     };
     std::map<long, BatchTune> batch_tune;
@@ -443,20 +451,26 @@ InstDev inst_dev(const Instance* in) {
 
 // where an instance's own shape keeps a slot's values and counters (Part)
 struct Places {
-    size_t at, by, count;
+    size_t at, count;
+    int stride;
 };
 template <typename T>
-Places places_of(const Instance* in, int slot, int p, int c) {
-    const InstDev I = inst_dev(in);
-    auto put = [&](auto part) { return Places{part.at(I, slot, p, c), (size_t)part.stride, part.count_at(I, slot, p, c)}; };
-    if (in->d.nstates == 4) switch (in->d.ncat) {
-        case 1: return put(Part<T, 4, 1>());
-        case 2: return put(Part<T, 4, 2>());
-        case 4: return put(Part<T, 4, 4>());
-        case 8: return put(Part<T, 4, 8>());
+Places places_of(const Instance* in, const InstDev& I, int slot, int p, int c) {
+    auto put = [&](auto part) {
+        return Places{part.at(I, slot, p, c), part.count_at(I, slot, p, c), part.stride};
+    };
+    auto states = [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        switch (in->d.ncat) {
+        case 1: return put(Part<T, N, 1>());
+        case 2: return put(Part<T, N, 2>());
+        case 4: return put(Part<T, N, 4>());
         }
-    const size_t pc = (size_t)p * in->d.ncat + c;
-    return Places{slot * I.slot_stride + pc * in->d.nstates, 1, slot * I.scale_stride + (in->d.safe_numeric ? pc : (size_t)p)};
+        return put(Part<T, N, 8>());
+    };
+    if (in->d.nstates == 4) return states(std::integral_constant<int, 4>());
+    if (in->d.nstates == kProtN) return states(std::integral_constant<int, kProtN>());
+    return states(std::integral_constant<int, kCodonN>());
 }
 
 ModelDev model_dev(const Instance* in) {
@@ -642,16 +656,24 @@ plk_status launch_traverse_mfma_c(plk_context* ctx, Instance* in, int nops, int 
                                   plk_end dad) {
     constexpr int N = 20;
     if (nops > 0) {
-        const int sub = ctx->mfma_sub;
-        const int grid = in->Ppad / (kMfmaTile * sub);
         const int pe = prof_begin(ctx);
-        auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), 0, ctx->stream, inst_dev(in), model_dev(in),
-                               in->ops, nops, reinterpret_cast<const T*>(in->tables), in->table_size);
-        };
-        if (sub == 4) go(k_traverse_mfma<T, N, C, 4>);
-        else if (sub == 2) go(k_traverse_mfma<T, N, C, 2>);
-        else go(k_traverse_mfma<T, N, C, 1>);
+        if constexpr (sizeof(T) == 8) {
+            const int waves = C == 8 ? 8 : 4;
+            const int grid = in->Ppad / (kProtPatterns * waves / C);
+            const size_t smem = prot_ops_smem(in->d.state_unknown, waves);
+            hipLaunchKernelGGL(k_traverse_prot<C>, dim3(grid), dim3(64 * waves), smem, ctx->stream, inst_dev(in),
+                               model_dev(in), in->tops, nops, reinterpret_cast<const T*>(in->tables), in->table_size);
+        } else {
+            const int sub = ctx->mfma_sub;
+            const int grid = in->Ppad / (kMfmaTile * sub);
+            auto go = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), 0, ctx->stream, inst_dev(in), model_dev(in),
+                                   in->ops, nops, reinterpret_cast<const T*>(in->tables), in->table_size);
+            };
+            if (sub == 4) go(k_traverse_mfma<T, N, C, 4>);
+            else if (sub == 2) go(k_traverse_mfma<T, N, C, 2>);
+            else go(k_traverse_mfma<T, N, C, 1>);
+        }
         HIP_TRY(hipGetLastError());
         prof_end(ctx, pe, K_TRAVERSE_MFMA, in->staged_bytes * in->d.npatterns,
                  in->staged_flops * in->d.npatterns);
@@ -755,7 +777,7 @@ plk_status stage_ops(plk_context* ctx, Instance* in, const plk_op* ops, int nops
         if (st != PLK_OK) return st;
         st = dmalloc(ctx, in, &in->tables, (size_t)(cap + 2) * 2 * in->table_size * elem);   // dna_ops reads two steps on
         if (st != PLK_OK) return st;
-        if (in->d.nstates == 4 && (st = dmalloc(ctx, in, &in->tops, sizeof(TileOp) * (cap + kTileAhead))) != PLK_OK) return st;
+        if (has_tile_ops(&in->d) && (st = dmalloc(ctx, in, &in->tops, sizeof(TileOp) * (cap + kTileAhead))) != PLK_OK) return st;
         in->ops_cap = cap;
     }
     std::vector<plk_op> stripped;
@@ -1129,7 +1151,7 @@ plk_status plk_instance_create(plk_context* ctx, const plk_instance_desc* d, int
     in->elem = d->precision == PLK_PREC_F32 ? 4 : 8;
     in->scale_elem = d->precision == PLK_PREC_F32 ? 4 : 2;
     in->sweep_table_size = (int)std::max(in->block * d->nstates, (size_t)(d->state_unknown + 1) * in->block);
-    in->table_size = d->nstates == kProtN ? prot_table_size(d->ncat, d->state_unknown)
+    in->table_size = d->nstates == kProtN ? prot_table_size(d->ncat, d->state_unknown, in->elem)
                      : d->nstates == 4  ? dna_table_size(d->ncat, d->state_unknown, in->elem)
                                         : in->sweep_table_size;
     const int n = d->nstates;
@@ -1711,12 +1733,14 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
     // first calls each run one candidate (fused or per-class launches x 1,
     // 2, 4, 8 workgroups per CU) and time it; results do not depend on the
     // shape, so no call repeats work. Batches of fewer tiles than a few per
-    // CU keep the default. Likely-good shapes first, so exploring costs little.
+    // CU keep the default: fused, as many workgroups as fit (90 partitions in
+    // FP32: 1071 us a call per class, two per CU; 938 fused). Likely-good shapes first,
+    // so exploring costs little.
     int lg = 0;
     while ((1 << lg) < total_tiles) lg++;
     const long key = (long)mix * 64 + lg;
-    int split = 1, bpc = ctx->batch_blocks_per_cu > 0 ? ctx->batch_blocks_per_cu : 2;
-    static const std::pair<int, int> kOrder[8] = {{1, 2}, {1, 4}, {0, 2}, {0, 4}, {1, 8}, {0, 8}, {1, 1}, {0, 1}};
+    int split = 0, bpc = ctx->batch_blocks_per_cu > 0 ? ctx->batch_blocks_per_cu : 4;
+    static const std::pair<int, int> kOrder[8] = {{0, 4}, {1, 4}, {0, 2}, {1, 2}, {0, 8}, {1, 8}, {0, 1}, {1, 1}};
     std::pair<int, int> cands[8];
     int ncand = 0;
     for (const auto& cd : kOrder)
@@ -1815,7 +1839,7 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
         b.tables = reinterpret_cast<const void*>(tab_bytes);   // offsets until the buffers exist
         tab_bytes += round_up((size_t)(items[i].nops + (b.n == 4 ? 2 : 0)) * 2 * in->table_size * in->elem, 256);
         b.tops = reinterpret_cast<const TileOp*>(tab_bytes);
-        if (b.n == 4) tab_bytes += round_up(sizeof(TileOp) * (size_t)(items[i].nops + kTileAhead), 256);
+        if (has_tile_ops(&in->d)) tab_bytes += round_up(sizeof(TileOp) * (size_t)(items[i].nops + kTileAhead), 256);
         b.root = reinterpret_cast<const double*>(root_doubles);
         root_doubles += (size_t)(in->d.state_unknown + 2) * in->block;
         const size_t item_smem = batch_smem_bytes(b.n, b.C, in->d.state_unknown, in->table_size, in->elem);
@@ -1896,7 +1920,8 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
         for (size_t k = 0; k < groups.size(); k++) {
             const Group& G = groups[k];
             const int pe2 = prof_begin(ctx);
-            const int fmask = __builtin_popcount(G.mask) > 1 ? BC_ALL : G.mask;   // fused DNA + protein
+            // fused DNA + protein: the classes of one storage, or any
+            const int fmask = __builtin_popcount(G.mask) == 1 || G.mask == BC_F64 || G.mask == BC_F32 ? G.mask : BC_ALL;
             const void* fn;
             switch (fmask) {
             case BC_DNA64: fn = (const void*)k_batch<BC_DNA64>; break;
@@ -1905,6 +1930,8 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
             case BC_PROT32: fn = (const void*)k_batch<BC_PROT32>; break;
             case BC_COD64: fn = (const void*)k_batch<BC_COD64>; break;
             case BC_COD32: fn = (const void*)k_batch<BC_COD32>; break;
+            case BC_F64: fn = (const void*)k_batch<BC_F64>; break;
+            case BC_F32: fn = (const void*)k_batch<BC_F32>; break;
             default: fn = (const void*)k_batch<BC_ALL>; break;
             }
             size_t smem = 0;
@@ -2760,14 +2787,15 @@ plk_status plk_read_partial(plk_context* ctx, int id, int slot, double* partial,
     // the copies hold this slot alone: places of an instance of one slot
     Instance one = *in;
     one.chunk_slots = 1;
+    const InstDev I = inst_dev(&one);
     const bool f64 = in->elem == 8;
     for (int p = 0; p < P; p++)
         for (int c = 0; c < C; c++) {
-            const Places at = f64 ? places_of<double>(&one, 0, p, c) : places_of<float>(&one, 0, p, c);
+            const Places at = f64 ? places_of<double>(in, I, 0, p, c) : places_of<float>(in, I, 0, p, c);
             if (partial)
                 for (int x = 0; x < n; x++)
-                    *partial++ = f64 ? reinterpret_cast<const double*>(hv.data())[at.at + x * at.by]
-                                     : (double)reinterpret_cast<const float*>(hv.data())[at.at + x * at.by];
+                    *partial++ = f64 ? reinterpret_cast<const double*>(hv.data())[at.at + x * at.stride]
+                                     : (double)reinterpret_cast<const float*>(hv.data())[at.at + x * at.stride];
             if (scale && (c == 0 || ncnt > 1))
                 *scale++ = in->scale_elem == 2 ? (int32_t)reinterpret_cast<const uint16_t*>(hc.data())[at.count]
                                                : reinterpret_cast<const int32_t*>(hc.data())[at.count];

@@ -129,23 +129,27 @@ __device__ inline ModelDev on_hbm(ModelDev m) {
 //   float    at 4l + x
 //   double   at [g / 2][x][j][g % 2] of pair l = j + 16g (j < 16): a lane's
 //            matrix operands, sixteen bytes at a time
+// 20 states in double storage: 32 patterns of a category make a block of 640
+// values, the operand registers of a wavefront's two sixteens side by side:
+// [x / 4][lane p % 16 + 16 (x % 4)][p / 16 % 2].
 template <typename T, int N, int C>
 struct Part {
-    static constexpr bool kLanes = N == 4 && sizeof(T) == 8;
-    static constexpr int stride = kLanes ? 32 : 1;
+    static constexpr bool kDna = N == 4, kProt = N == 20 && sizeof(T) == 8, kLanes = kDna && sizeof(T) == 8;
+    static constexpr int stride = kLanes || kProt ? 32 : 1;
     __host__ __device__ static size_t at(const InstDev& I, int slot, int p, int c) {
-        if (N != 4) return slot * I.slot_stride + (size_t)p * (N * C) + c * N;
+        if (kProt) return slot * I.slot_stride + ((size_t)(p >> 5) * C + c) * 640 + (p & 15) * 2 + (p >> 4 & 1);
+        if (!kDna) return slot * I.slot_stride + (size_t)p * (N * C) + c * N;
         const int l = pair(p, c);
         const int in = kLanes ? (l >> 5) * 128 + (l & 15) * 2 + (l >> 4 & 1) : l * 4;
         return ((size_t)(p / (64 / C)) * I.chunk_slots + slot) * 256 + in;
     }
     __host__ __device__ static size_t count_at(const InstDev& I, int slot, int p, int c) {
-        if (N != 4) return slot * I.scale_stride + (I.safe ? (size_t)p * C + c : (size_t)p);
+        if (!kDna) return slot * I.scale_stride + (I.safe ? (size_t)p * C + c : (size_t)p);
         return ((size_t)(p / (64 / C)) * I.chunk_slots + slot) * 64 + pair(p, c);
     }
     __host__ __device__ static int pair(int p, int c) { return (p % (64 / C) >> 2) * (4 * C) + 4 * c + (p & 3); }
     // the thread of (p, c) writes a counter of its own
-    __device__ static bool counts(const InstDev& I, int c) { return N == 4 || I.safe || c == 0; }
+    __device__ static bool counts(const InstDev& I, int c) { return kDna || I.safe || c == 0; }
 };
 
 // Elements of one (op, child) table for 4 states. Double storage: a child's
@@ -175,11 +179,26 @@ constexpr int kProtN = 20;                 // protein states
 constexpr int kProtKSteps = 5;             // 4-wide K steps over 20 states
 constexpr int kProtFrag = 2 * kProtKSteps * 64;   // fragment elements per category
 
-// Elements of one (op, child) table for 20 states: an internal child in
-// fragment order (C categories), a tip child's lookup [SU+1][C][20].
-__host__ __device__ inline int prot_table_size(int C, int SU) {
+// Elements of one (op, child) table for 20 states. Float storage: an internal
+// child in fragment order (C categories), a tip child's lookup [SU+1][C][20].
+// Double storage: a step's are [C][2 children][kProtKid], an internal child's
+// matrix as 4x4 blocks (prot_ops), a tip child's lookup [SU+1][20], or its
+// matrix if the lookup is larger than kProtKid.
+constexpr int kProtBlocks = 13 * 32;      // 25 blocks of 16, in pairs
+constexpr int kProtKid = 512;
+__host__ __device__ inline bool prot_lut(int SU) { return (SU + 1) * kProtN <= kProtKid; }
+__host__ __device__ inline int prot_table_size(int C, int SU, size_t elem) {
     const int frag = C * kProtFrag, lut = (SU + 1) * C * kProtN;
-    return frag > lut ? frag : lut;
+    return elem == 8 ? C * kProtKid : frag > lut ? frag : lut;
+}
+// A 20x20 matrix as blocks B of 4x4, each two at [B / 2][x % 4 + 4 (k % 4)][B % 2],
+// in the order in which prot_ops multiplies: the rows X = x / 4 two at a time
+// along K = k / 4, then the fifth. The (x, k) of element t, x = -1 past the last.
+__host__ __device__ inline void prot_block_index(int t, int& x, int& k) {
+    const int B = 2 * (t >> 5) + (t & 1), e = t >> 1 & 15;
+    const int X = B >= 20 ? 4 : B / 10 * 2 + B % 2, K = B >= 20 ? B - 20 : B % 10 / 2;
+    x = B < 25 ? 4 * X + (e & 3) : -1;
+    k = 4 * K + (e >> 2);
 }
 
 // Fragment order of an internal child's table, per category:
@@ -204,12 +223,12 @@ k_copy(const double4* __restrict__ src, double4* __restrict__ dst, size_t n) {
 enum TraverseMode { MODE_PARTIALS = 0, MODE_BRANCH = 1, MODE_THETA = 2 };
 enum BufferMode { BUF_DERV = 0, BUF_LNL = 1 };
 
-// One traversal step for dna_ops (4 states): three scalar loads of sixteen
-// bytes, each made when its part of the step is due.
+// One traversal step for dna_ops and prot_ops: scalar loads of sixteen bytes,
+// each made when its part of the step is due.
 struct alignas(64) TileOp {
     uint64_t tip[2];      // a tip child's row of states (others: taxon 0's)
     uint32_t v[2], sc[2]; // a slot child's values and counters, kNoSlot for one that comes from elsewhere
-    uint32_t dst, dsc;    // the dad's; offsets in bytes from the chunk's slot 0 (far instances: slots)
+    uint32_t dst, dsc;    // the dad's; offsets in bytes from the chunk's slot 0 (far instances and 20 states: slots)
     uint32_t kind;        // of child k in bits 2k and 2k + 1, below
     uint32_t root;        // bit k: child k is the root leaf (state-basis models)
 };
@@ -233,13 +252,13 @@ __device__ inline void make_tile_op(const InstDev& I, const plk_op* __restrict__
                                     unsigned root = 0) {
     const plk_op op = ops[o];
     const int last = o > 0 ? ops[o - 1].dad_slot : -1, last2 = o > 1 ? ops[o - 2].dad_slot : -1;
-    const bool far = dna_far(I.chunk_slots, sizeof(T));
+    const bool far = I.n != 4 || dna_far(I.chunk_slots, sizeof(T));
     const uint32_t nv = far ? 1 : kChunkValues<T>, nc = far ? 1 : kChunkCounts<T>;
     TileOp t;
     t.kind = 0;
     for (int k = 0; k < 2; k++) {
         const int id = op.child[k].id;
-        const int kind = op.child[k].is_tip ? CHILD_TIP : id == last ? CHILD_LAST : id == last2 ? CHILD_LAST2 : CHILD_SLOT;
+        const int kind = op.child[k].is_tip ? CHILD_TIP : id == last ? CHILD_LAST : id == last2 && I.n == 4 ? CHILD_LAST2 : CHILD_SLOT;
         t.kind |= kind << 2 * k;
         t.tip[k] = reinterpret_cast<uint64_t>(I.states) + (kind == CHILD_TIP ? (size_t)id * I.Ppad : 0);
         t.v[k] = kind == CHILD_SLOT ? id * nv : kNoSlot;
@@ -259,7 +278,7 @@ __device__ inline void make_tile_op(const InstDev& I, const plk_op* __restrict__
 // for an internal child, or the tip table leaf[s][c][x] =
 // sum_i echild[c][x][i] tip[s][i] (leaf[SU] = 1) for a tip child.
 // One workgroup per (op, child, category); tables are written in storage
-// precision. 4 states: also the steps' addresses (tops).
+// precision. 4 states, and 20 in double storage: also the steps' TileOps.
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
 k_prep_ops(const plk_op* __restrict__ ops, int nops, ModelDev m, int n, int C, int SU,
@@ -274,8 +293,18 @@ k_prep_ops(const plk_op* __restrict__ ops, int nops, ModelDev m, int n, int C, i
     double* ex = sh;
     for (int i = threadIdx.x; i < n; i += blockDim.x) ex[i] = exp(m.eval[i] * (m.rates[c] * ch.length));
     T* out = tables + (size_t)(2 * o + k) * table_size;
-    if (!ch.is_tip || (n == 4 && sizeof(T) == 8)) {
+    T* kid = tables + (size_t)2 * o * table_size + (2 * c + k) * kProtKid;   // 20 states, double storage
+    const bool tip_matrix = sizeof(T) == 8 && (n == 4 || (n == kProtN && !prot_lut(SU)));
+    if (!ch.is_tip || tip_matrix) {
         __syncthreads();
+        if (n == kProtN && sizeof(T) == 8) {
+            for (int t = threadIdx.x; t < kProtBlocks; t += blockDim.x) {
+                int x, i;
+                prot_block_index(t, x, i);
+                kid[t] = x < 0 ? (T)0 : (T)(m.evec[x * n + i] * ex[i]);
+            }
+            return;
+        }
         if (n == kProtN) {
             // the matrix-core tile's fragment order
             T* oc = out + (size_t)c * kProtFrag;
@@ -317,7 +346,8 @@ k_prep_ops(const plk_op* __restrict__ ops, int nops, ModelDev m, int n, int C, i
             v = ev[0] * ex[0] * tp[0];
             for (int i = 1; i < n; i++) v += ev[i] * ex[i] * tp[i];
         }
-        out[(size_t)(s * C + c) * n + x] = (T)v;
+        if (n == kProtN && sizeof(T) == 8) kid[t] = (T)v;
+        else out[(size_t)(s * C + c) * n + x] = (T)v;
     }
 }
 

@@ -1,6 +1,7 @@
 // Partial-likelihood updates for protein (20 states) on the matrix cores:
 // tree/phylokernelnew.h:1632-2031 as two contractions per category and
-// traversal step,
+// traversal step. Double storage: prot_ops, at the end. Float storage
+// (prot_ops_tile):
 //   phase A  tmp[x][p] = prod_children sum_k E_child[c][x][k] * child[p][c][k]
 //            (tip children: the lookup leaf[s_p][c][x])
 //   phase B  dad[p][i] = sum_x tmp[p][x] * inv_evec[i][x]
@@ -267,10 +268,252 @@ template <typename T, int N, int C, int SUB>
 __global__ void __launch_bounds__(kThreads)
 k_traverse_mfma(InstDev I, ModelDev m, const plk_op* __restrict__ ops, int nops,
                 const T* __restrict__ tables, int table_size) {
-    static_assert(N == kProtN, "20-state tile");
+    static_assert(N == kProtN && sizeof(T) == 4, "20-state tile of float storage");
     __shared__ T mx_sh[prot_mx_elems<C, SUB>()];
     prot_ops_tile<T, C, SUB>(I, m.inv_evec, ops, nops, tables, table_size, mx_sh,
                              blockIdx.x * kMfmaTile * SUB);
+}
+
+// ---------------------------------------------------------------------------
+// Double storage. What bounded the 16x16x4 tile: thirty vector memory
+// instructions a step for 16 patterns of a category (each child's matrix from
+// L2 for every 16 patterns, operands and results in scattered rows, the lookup
+// rows of a tip), the memory path of a CU busy 92% of the time, and of its
+// 16x16 products of 20 states a third padding. Here
+//   - a product of 20 states is 25 products of 4x4x4 (v_mfma_f64_4x4x4, four
+//     blocks: the same matrix block, sixteen patterns), with no padding, and
+//     its result is laid out as its operand: register X of lane q + 16k holds
+//     value 4X + k of pattern q. Two sixteens a wavefront share each block;
+//   - slots are stored as these registers (Part): whole lines, five accesses
+//     of a kilobyte for 32 patterns;
+//   - the last dad stays in registers (of a random tree, three of four child
+//     reads);
+//   - a category's tables of the next step are loaded as 8 KB in order while
+//     this one runs, and read from LDS, as is U^-1.
+// A wavefront owns a category; the only exchange is a mask of the patterns
+// that are below the rescale threshold in it, one barrier a step (normal mode).
+// 100 taxa x 20,000 patterns x 4 categories: 969 -> 448 us (3.1 TB/s with the
+// one slot in four re-read; 470 with waits for copies of children in flight,
+// 568 in 200 registers, two waves a SIMD; the protein
+// tiles of 500 partitions in a batch 3313 -> 2370 us). Bound now by the step's chain of products and
+// exchange, 2.2 us of a lone wavefront, at 2.4 wavefronts a SIMD.
+constexpr int kProtPatterns = 32;          // of a wavefront
+
+// LDS: U^-1 | tip vectors and (1, 0, ...) for the root leaf, whose matrix holds
+// the frequencies in column 0, if read | each wavefront's tables of a step | masks [2][waves]
+__host__ __device__ inline size_t prot_ops_smem(int SU, int waves) {
+    return (kProtBlocks + (prot_lut(SU) ? 0 : (size_t)(SU + 2) * kProtN) + (size_t)waves * 2 * kProtKid) * 8 + 2 * waves * 4;
+}
+
+// the workgroup's waves take categories, then blocks of 32 patterns from
+// p_first. Three waves a SIMD (140 registers): at four (128) the spills' reloads
+// wait for every load in flight.
+template <int C>
+__device__ inline void prot_ops(const InstDev& I, const ModelDev& m, const TileOp* tops, int nops,
+                                const double* tables, int table_size, int p_first, unsigned char* smem) {
+    constexpr int kSets = 2, kX = 5, kVec = 2 * kProtKid / 128;   // sixteens; blocks of a state range; a step's loads
+    if (nops == 0) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = blockDim.x >> 6;
+    const int c = wave % C, p0 = p_first + wave / C * kProtPatterns;
+    double* inv_sh = reinterpret_cast<double*>(smem);
+    double* tip_sh = inv_sh + kProtBlocks;
+    const bool lut = prot_lut(I.SU);
+    double* all_sh = tip_sh + (lut ? 0 : (I.SU + 2) * kProtN);
+    double* e_sh = all_sh + wave * 2 * kProtKid;
+    unsigned* mask_sh = reinterpret_cast<unsigned*>(all_sh + waves * 2 * kProtKid);
+    __syncthreads();
+    for (int t = threadIdx.x; t < kProtBlocks; t += blockDim.x) {
+        int x, k;
+        prot_block_index(t, x, k);
+        inv_sh[t] = x < 0 ? 0.0 : m.inv_evec[x * kProtN + k];
+    }
+    if (!lut)
+        for (int t = threadIdx.x, n = (I.SU + 1) * kProtN; t < n + kProtN; t += blockDim.x)
+            tip_sh[t] = t < n ? m.tip[t] : t == n ? 1.0 : 0.0;
+    __syncthreads();
+    const bool safe = I.safe != 0;
+    const int pl = lane & 31;                       // lane l keeps the counter of pattern p0 + l % 32
+    const unsigned no_invar = (unsigned)__builtin_amdgcn_ballot_w64(I.invar[p0 + pl] == 0.0);
+    const int q = lane & 15, k = lane >> 4;
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const uint64_t vbase = (uint64_t)I.partial + ((size_t)(p0 >> 5) * C + c) * (640 * 8);
+    const uint64_t vstride = I.slot_stride * 8;
+    Hbm<uint16_t>* counts = (Hbm<uint16_t>*)I.scale + (safe ? (size_t)p0 * C + c : (size_t)p0);
+    const int sat = safe ? pl * C : pl;
+    const bool counting = safe || c == 0;           // normal mode: one counter a pattern
+
+    struct Vec {   // [X][sixteen]
+        d2 v[kX];
+    };
+    auto load_slot = [&](uint32_t slot, Vec& to) {
+        const Hbm<d2>* from = (const Hbm<d2>*)(vbase + slot * vstride) + lane;
+#pragma unroll
+        for (int X = 0; X < kX; X++) to.v[X] = from[64 * X];
+    };
+    // a matrix in LDS times both sixteens, two rows of blocks at a time:
+    // four chains of products in flight, and few registers
+    const int at = ((lane & 3) + 4 * k) * 2;
+    auto mul = [&](const double* blocks, const Vec& b, auto put) {
+        auto block2 = [&](int B2) { return *reinterpret_cast<const d2*>(blocks + B2 * 32 + at); };
+        auto fma4 = [&](double a, double v, double d) { return __builtin_amdgcn_mfma_f64_4x4x4f64(a, v, d, 0, 0, 0); };
+#pragma unroll
+        for (int X = 0; X < 4; X += 2) {
+            double d[2][kSets] = {};
+#pragma unroll
+            for (int K = 0; K < kX; K++) {
+                const d2 a = block2(X / 2 * 5 + K);
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int s = 0; s < kSets; s++) d[h][s] = fma4(a[h], b.v[K][s], d[h][s]);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int s = 0; s < kSets; s++) put(s, X + h, d[h][s]);
+            __builtin_amdgcn_sched_barrier(0);   // no reads further ahead: registers
+        }
+        double d[kSets] = {};
+#pragma unroll
+        for (int K = 0; K < kX; K++) {
+            const d2 a = block2(10 + K / 2);
+#pragma unroll
+            for (int s = 0; s < kSets; s++) d[s] = fma4(a[K & 1], b.v[K][s], d[s]);
+        }
+#pragma unroll
+        for (int s = 0; s < kSets; s++) put(s, 4, d[s]);
+    };
+
+    const uint64_t tp = (uint64_t)tops;
+    const Hbm<tile_u4>* tab = (const Hbm<tile_u4>*)((const Hbm<double>*)tables + 2 * c * kProtKid);
+    tile_u4 e_next[kVec];
+    auto load_tables = [&]() {
+#pragma unroll
+        for (int r = 0; r < kVec; r++) e_next[r] = tab[lane + 64 * r];
+    };
+    struct Kid : Vec {
+        int st[kSets], sc;
+        __device__ Kid() {}
+    } kid[2];
+    Vec last;
+    int sc_last = 0;
+    auto load_kids = [&](uint64_t op, bool first) {
+        const tile_u4 tips = load_u4(op), kids = load_u4(op + 16), end = load_u4(op + 32);
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const unsigned kind = end[2] >> 2 * j & 3;
+            kid[j] = Kid();   // the last step's ends here, also where no load replaces it
+            if (kind == CHILD_TIP) {
+                const Hbm<uint8_t>* row = (const Hbm<uint8_t>*)((uint64_t)tips[2 * j + 1] << 32 | tips[2 * j]) + p0;
+#pragma unroll
+                for (int s = 0; s < kSets; s++) kid[j].st[s] = row[16 * s + q];
+            }
+            unsigned matrix = lut ? CHILD_LAST : kind, slots = kind;
+            asm("" : "+s"(matrix));
+            if (matrix == CHILD_TIP) {
+                kid[j].sc = 0;
+#pragma unroll
+                for (int s = 0; s < kSets; s++) {
+                    const double* row = tip_sh + (end[3] >> j & 1 ? I.SU + 1 : kid[j].st[s]) * kProtN + k;
+#pragma unroll
+                    for (int K = 0; K < kX; K++) kid[j].v[K][s] = row[4 * K];
+                }
+            }
+            asm("" : "+s"(slots));   // ifs, not a switch, whose joins would copy what is being loaded
+            if (slots == CHILD_SLOT || (first && matrix != CHILD_TIP)) {
+                const uint32_t slot = slots == CHILD_SLOT ? kids[j] : 0;
+                load_slot(slot, kid[j]);
+                kid[j].sc = counts[(size_t)slot * I.scale_stride + sat];
+            }
+        }
+    };
+    load_tables();
+    // unconditionally, after the tables: the loop's first wait for them must
+    // not be shorter than the later ones, which have stores to look past
+    load_kids(tp, true);
+    for (int o = 0; o < nops; o++) {
+        const uint64_t op = tp + (uint64_t)o * sizeof(TileOp);
+        const tile_u4 end = load_u4(op + 32);
+        const unsigned kinds = end[2];
+#pragma unroll
+        for (int r = 0; r < kVec; r++)
+            *(reinterpret_cast<tile_u4*>(e_sh) + lane + 64 * r) = e_next[r];
+        Vec f;
+        int sc = 0;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const unsigned kind = kinds >> 2 * j & 3;
+            const double* e = e_sh + j * kProtKid;
+            auto put = [&](int s, int X, double v) { f.v[X][s] = j == 0 ? v : f.v[X][s] * v; };
+            if (kind == CHILD_TIP && lut) {
+#pragma unroll
+                for (int s = 0; s < kSets; s++)
+#pragma unroll
+                    for (int X = 0; X < kX; X++) put(s, X, e[kid[j].st[s] * kProtN + 4 * X + k]);
+            } else if (kind == CHILD_LAST) {
+                mul(e, last, put);
+                sc += sc_last;
+            } else {
+                mul(e, kid[j], put);
+                sc += kid[j].sc;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // the next step's, after the last one its own again: a condition would
+        // keep the old values in registers through the step
+        const int ahead = o + 1 < nops;
+        tab += ahead * table_size;   // 2 * table_size values
+        load_tables();
+        mul(inv_sh, f, [&](int s, int X, double v) { last.v[X][s] = v; });
+        // patterns with every value below the threshold, in all categories in normal mode
+        unsigned small = 0;
+#pragma unroll
+        for (int s = 0; s < kSets; s++) {
+            double mx = 0.0;
+#pragma unroll
+            for (int X = 0; X < kX; X++) mx = fmax(mx, fabs(last.v[X][s]));
+            unsigned long long b = __builtin_amdgcn_ballot_w64(mx < Prec<double>::threshold);
+            b &= b >> 32;
+            b &= b >> 16;
+            small |= (unsigned)(b & 0xffff) << 16 * s;
+        }
+        if (!safe) {
+            unsigned* masks = mask_sh + (o & 1) * waves;
+            if (lane == 0) masks[wave] = small;
+            __syncthreads();
+            small = ~0u;
+#pragma unroll
+            for (int w = 0; w < C; w++) small &= masks[wave / C * C + w];
+            small = __builtin_amdgcn_readfirstlane(small);
+        }
+        small &= no_invar;
+        if (small && kinds != (CHILD_TIP | CHILD_TIP << 2)) {
+            int l = lane;
+            asm("" : "+v"(l));   // rare: no masks kept in registers for it
+#pragma unroll
+            for (int s = 0; s < kSets; s++)
+                if (small >> (16 * s + (l & 15)) & 1)
+#pragma unroll
+                    for (int X = 0; X < kX; X++) last.v[X][s] = Prec<double>::apply(last.v[X][s], 1);
+            sc += small >> (l & 31) & 1;
+        }
+        sc_last = sc;
+        load_kids(op + ahead * sizeof(TileOp), false);
+        Hbm<d2>* to = (Hbm<d2>*)(vbase + end[0] * vstride) + lane;
+#pragma unroll
+        for (int X = 0; X < kX; X++) to[64 * X] = last.v[X];
+        if (counting && lane < 32) counts[(size_t)end[0] * I.scale_stride + sat] = (uint16_t)sc;
+    }
+}
+
+// workgroups of eight waves for eight categories
+template <int C>
+__global__ void __launch_bounds__(C == 8 ? 512 : kThreads, 3)
+k_traverse_prot(InstDev I, ModelDev m, const TileOp* __restrict__ tops, int nops, const double* __restrict__ tables,
+                int table_size) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    prot_ops<C>(I, m, tops, nops, tables, table_size, blockIdx.x * (kProtPatterns * (C < 4 ? 4 / C : 1)), smem);
 }
 
 }  // namespace plkdev

@@ -89,6 +89,17 @@ k_nr_prep_ops(const plk_op* __restrict__ ops, const uint8_t* __restrict__ flags,
         }
         return;
     }
+    const bool prot = n == kProtN && sizeof(T) == 8;
+    T* kid = tables + (size_t)2 * o * table_size + (2 * c + k) * kProtKid;
+    if (prot && (!ch.is_tip || !prot_lut(SU))) {
+        for (int t = threadIdx.x; t < kProtBlocks; t += blockDim.x) {
+            int x, i;
+            prot_block_index(t, x, i);
+            kid[t] = x < 0 ? (T)0 : fl & kNrRootLeaf ? (i == 0 ? (T)D.pi[(size_t)m * n + x] : (T)0)
+                                                    : (T)(tr ? P[i * n + x] : P[x * n + i]);
+        }
+        return;
+    }
     if (!ch.is_tip) {
         if (n == kProtN) {
             T* oc = out + (size_t)c * kProtFrag;
@@ -117,7 +128,8 @@ k_nr_prep_ops(const plk_op* __restrict__ ops, const uint8_t* __restrict__ flags,
             v = 0.0;
             for (int y = 0; y < n; y++) v += (tr ? P[y * n + x] : P[x * n + y]) * tip[s * n + y];
         }
-        out[(size_t)(s * C + c) * n + x] = (T)v;
+        if (prot) kid[t] = (T)v;
+        else out[(size_t)(s * C + c) * n + x] = (T)v;
     }
 }
 
