@@ -185,10 +185,10 @@ __device__ inline double branch_end_stream(const InstDev& I, plk_end node, plk_e
         if (dad.is_tip) {
             const double* tp = tip_eig + s * N;
 #pragma unroll 4
-            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i * L::stride] * tp[i] * adjust);
+            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[L::x(p, i)] * tp[i] * adjust);
         } else {
 #pragma unroll 4
-            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i * L::stride] * (double)dv[i * L::stride] * adjust);
+            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[L::x(p, i)] * (double)dv[L::x(p, i)] * adjust);
         }
         if (c == 0) I.buffer_scale[p] = (double)minsc * Prec<T>::log_unit;
         return 0.0;
@@ -198,12 +198,12 @@ __device__ inline double branch_end_stream(const InstDev& I, plk_end node, plk_e
         const double* lut = root_sh + block + (s * C + c) * N;
         lhc = lut[0] * (double)nv[0];
 #pragma unroll 1
-        for (int i = 1; i < N; i++) lhc = fma(lut[i], (double)nv[i * L::stride], lhc);
+        for (int i = 1; i < N; i++) lhc = fma(lut[i], (double)nv[L::x(p, i)], lhc);
     } else {
         const double* val = root_sh + c * N;
         lhc = val[0] * (double)dv[0] * (double)nv[0];
 #pragma unroll 1
-        for (int i = 1; i < N; i++) lhc = fma(val[i] * (double)dv[i * L::stride], (double)nv[i * L::stride], lhc);
+        for (int i = 1; i < N; i++) lhc = fma(val[i] * (double)dv[L::x(p, i)], (double)nv[L::x(p, i)], lhc);
     }
     if (minsc_out) *minsc_out = minsc;
     return safe ? group_sum_sumvec<C>(lhc * adjust) : group_sum_ordered<C>(lhc);

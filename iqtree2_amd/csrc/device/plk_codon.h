@@ -272,9 +272,9 @@ k_root_stream(InstDev I, ModelDev m, int mode, plk_end node, plk_end dad,
         T* th = reinterpret_cast<T*>(I.theta) + (size_t)p * block + c * N;
         if (dad.is_tip) {
             const double* tp = m.tip + s * N;
-            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i * L::stride] * tp[i] * adjust);
+            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[L::x(p, i)] * tp[i] * adjust);
         } else {
-            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[i * L::stride] * (double)dv[i * L::stride] * adjust);
+            for (int i = 0; i < N; i++) th[i] = (T)((double)nv[L::x(p, i)] * (double)dv[L::x(p, i)] * adjust);
         }
         if (c == 0) I.buffer_scale[p] = (double)minsc * Prec<T>::log_unit;
         return;
@@ -283,11 +283,11 @@ k_root_stream(InstDev I, ModelDev m, int mode, plk_end node, plk_end dad,
     if (dad.is_tip) {
         const double* lut = root_tab + block + (size_t)(s * C + c) * N;
         lhc = lut[0] * (double)nv[0];
-        for (int i = 1; i < N; i++) lhc = fma(lut[i], (double)nv[i * L::stride], lhc);
+        for (int i = 1; i < N; i++) lhc = fma(lut[i], (double)nv[L::x(p, i)], lhc);
     } else {
         const double* val = root_tab + c * N;
         lhc = val[0] * (double)dv[0] * (double)nv[0];
-        for (int i = 1; i < N; i++) lhc = fma(val[i] * (double)dv[i * L::stride], (double)nv[i * L::stride], lhc);
+        for (int i = 1; i < N; i++) lhc = fma(val[i] * (double)dv[L::x(p, i)], (double)nv[L::x(p, i)], lhc);
     }
     const double lh0 = safe ? group_sum_sumvec<C>(lhc * adjust) : group_sum_ordered<C>(lhc);
     double contrib = 0.0;

@@ -452,12 +452,14 @@ InstDev inst_dev(const Instance* in) {
 // where an instance's own shape keeps a slot's values and counters (Part)
 struct Places {
     size_t at, count;
-    int stride;
+    int x[kCodonN];
 };
 template <typename T>
 Places places_of(const Instance* in, const InstDev& I, int slot, int p, int c) {
     auto put = [&](auto part) {
-        return Places{part.at(I, slot, p, c), part.count_at(I, slot, p, c), part.stride};
+        Places r{part.at(I, slot, p, c), part.count_at(I, slot, p, c), {}};
+        for (int i = 0; i < in->d.nstates; i++) r.x[i] = part.x(p, i);
+        return r;
     };
     auto states = [&](auto n) {
         constexpr int N = decltype(n)::value;
@@ -2794,8 +2796,8 @@ plk_status plk_read_partial(plk_context* ctx, int id, int slot, double* partial,
             const Places at = f64 ? places_of<double>(in, I, 0, p, c) : places_of<float>(in, I, 0, p, c);
             if (partial)
                 for (int x = 0; x < n; x++)
-                    *partial++ = f64 ? reinterpret_cast<const double*>(hv.data())[at.at + x * at.stride]
-                                     : (double)reinterpret_cast<const float*>(hv.data())[at.at + x * at.stride];
+                    *partial++ = f64 ? reinterpret_cast<const double*>(hv.data())[at.at + at.x[x]]
+                                     : (double)reinterpret_cast<const float*>(hv.data())[at.at + at.x[x]];
             if (scale && (c == 0 || ncnt > 1))
                 *scale++ = in->scale_elem == 2 ? (int32_t)reinterpret_cast<const uint16_t*>(hc.data())[at.count]
                                                : reinterpret_cast<const int32_t*>(hc.data())[at.count];

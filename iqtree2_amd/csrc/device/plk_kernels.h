@@ -116,7 +116,7 @@ __device__ inline ModelDev on_hbm(ModelDev m) {
 }
 
 // Where slot s keeps value x of (pattern p, category c), element
-// at(I, s, p, c) + x * stride, and its counter, element count_at(I, s, p, c)
+// at(I, s, p, c) + x(p, x), and its counter, element count_at(I, s, p, c)
 // ([slot][p], safe mode [slot][p][c]; 4 states one per pair in both modes, so
 // that a wavefront writes whole lines).
 // 4 states: 64 (pattern, category) pairs, those of 64 / C adjacent patterns,
@@ -130,18 +130,26 @@ __device__ inline ModelDev on_hbm(ModelDev m) {
 //   double   at [g / 2][x][j][g % 2] of pair l = j + 16g (j < 16): a lane's
 //            matrix operands, sixteen bytes at a time
 // 20 states in double storage: 32 patterns of a category make a block of 640
-// values, the operand registers of a wavefront's two sixteens side by side:
-// [x / 4][lane p % 16 + 16 (x % 4)][p / 16 % 2].
+// values, the operand registers X = x / 4 of a wavefront's two sixteens S, two
+// side by side: [(S0, X0 X1), (S0, X2 X3), the same of S1, (X4, S0 S1)]
+// [lane p % 16 + 16 (x % 4)][2], so that a thread of its own (p, c) reads two
+// values at a time, too (a sweep of 20 taxa x 1,200 sites with the sixteens
+// side by side, one at a time: 2319 us, so: 2170; traversal 448 and 442 us).
 template <typename T, int N, int C>
 struct Part {
     static constexpr bool kDna = N == 4, kProt = N == 20 && sizeof(T) == 8, kLanes = kDna && sizeof(T) == 8;
-    static constexpr int stride = kLanes || kProt ? 32 : 1;
     __host__ __device__ static size_t at(const InstDev& I, int slot, int p, int c) {
-        if (kProt) return slot * I.slot_stride + ((size_t)(p >> 5) * C + c) * 640 + (p & 15) * 2 + (p >> 4 & 1);
+        if (kProt) return slot * I.slot_stride + ((size_t)(p >> 5) * C + c) * 640 + (p >> 4 & 1) * 256 + (p & 15) * 2;
         if (!kDna) return slot * I.slot_stride + (size_t)p * (N * C) + c * N;
         const int l = pair(p, c);
         const int in = kLanes ? (l >> 5) * 128 + (l & 15) * 2 + (l >> 4 & 1) : l * 4;
         return ((size_t)(p / (64 / C)) * I.chunk_slots + slot) * 256 + in;
+    }
+    // value i, from at(), where value 0 is
+    __host__ __device__ static int x(int p, int i) {
+        if (kProt && i < 16) return (i >> 3) * 128 + (i & 3) * 32 + (i >> 2 & 1);
+        if (kProt) return 512 - 255 * (p >> 4 & 1) + (i & 3) * 32;
+        return kLanes ? 32 * i : i;
     }
     __host__ __device__ static size_t count_at(const InstDev& I, int slot, int p, int c) {
         if (!kDna) return slot * I.scale_stride + (I.safe ? (size_t)p * C + c : (size_t)p);
@@ -550,7 +558,7 @@ __device__ inline void op_load(const InstDev& I, int l_tip, int l_id, int r_tip,
     } else {
         const T* src = partial + Part<T, N, C>::at(I, l_id, p, c);
 #pragma unroll
-        for (int i = 0; i < N; i++) in.l[i] = src[i * Part<T, N, C>::stride];
+        for (int i = 0; i < N; i++) in.l[i] = src[Part<T, N, C>::x(p, i)];
         in.scl = scale[Part<T, N, C>::count_at(I, l_id, p, c)];
     }
     if (r_tip) {
@@ -558,7 +566,7 @@ __device__ inline void op_load(const InstDev& I, int l_tip, int l_id, int r_tip,
     } else {
         const T* src = partial + Part<T, N, C>::at(I, r_id, p, c);
 #pragma unroll
-        for (int i = 0; i < N; i++) in.r[i] = src[i * Part<T, N, C>::stride];
+        for (int i = 0; i < N; i++) in.r[i] = src[Part<T, N, C>::x(p, i)];
         in.scr = scale[Part<T, N, C>::count_at(I, r_id, p, c)];
     }
 }
@@ -623,7 +631,7 @@ __device__ inline void op_finish(const InstDev& I, const T* inv_sh, const T* tL,
     }
     T* dst = partial + Part<T, N, C>::at(I, dad_slot, p, c);
 #pragma unroll
-    for (int i = 0; i < N; i++) dst[i * Part<T, N, C>::stride] = dadv[i];
+    for (int i = 0; i < N; i++) dst[Part<T, N, C>::x(p, i)] = dadv[i];
     if (Part<T, N, C>::counts(I, c)) scale[Part<T, N, C>::count_at(I, dad_slot, p, c)] = (ST)sc;
 }
 
@@ -1060,7 +1068,7 @@ __device__ inline void load_branch(const InstDev& I, plk_end node, plk_end dad, 
     const bool safe = I.safe != 0;
     const T* nsrc = partial + Part<T, N, C>::at(I, node.id, p, c);
 #pragma unroll
-    for (int i = 0; i < N; i++) nv[i] = (double)nsrc[i * Part<T, N, C>::stride];
+    for (int i = 0; i < N; i++) nv[i] = (double)nsrc[Part<T, N, C>::x(p, i)];
     int sc = scale[Part<T, N, C>::count_at(I, node.id, p, c)];
     if (dad.is_tip) {
         if (tip_sh) {   // callers that use a val-weighted lookup pass nullptr
@@ -1072,7 +1080,7 @@ __device__ inline void load_branch(const InstDev& I, plk_end node, plk_end dad, 
     } else {
         const T* dsrc = partial + Part<T, N, C>::at(I, dad.id, p, c);
 #pragma unroll
-        for (int i = 0; i < N; i++) dv[i] = (double)dsrc[i * Part<T, N, C>::stride];
+        for (int i = 0; i < N; i++) dv[i] = (double)dsrc[Part<T, N, C>::x(p, i)];
         sc += scale[Part<T, N, C>::count_at(I, dad.id, p, c)];
     }
     minsc = sc;

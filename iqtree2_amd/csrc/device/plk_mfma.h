@@ -343,8 +343,13 @@ __device__ inline void prot_ops(const InstDev& I, const ModelDev& m, const TileO
     const int sat = safe ? pl * C : pl;
     const bool counting = safe || c == 0;           // normal mode: one counter a pattern
 
-    struct Vec {   // [X][sixteen]
+    struct Vec {   // registers X of sixteens s, in the order of a slot
         d2 v[kX];
+        __device__ double operator()(int X, int s) const { return X < 4 ? v[2 * s + X / 2][X & 1] : v[4][s]; }
+        __device__ void set(int X, int s, double w) {
+            if (X < 4) v[2 * s + X / 2][X & 1] = w;
+            else v[4][s] = w;
+        }
     };
     auto load_slot = [&](uint32_t slot, Vec& to) {
         const Hbm<d2>* from = (const Hbm<d2>*)(vbase + slot * vstride) + lane;
@@ -366,7 +371,7 @@ __device__ inline void prot_ops(const InstDev& I, const ModelDev& m, const TileO
 #pragma unroll
                 for (int h = 0; h < 2; h++)
 #pragma unroll
-                    for (int s = 0; s < kSets; s++) d[h][s] = fma4(a[h], b.v[K][s], d[h][s]);
+                    for (int s = 0; s < kSets; s++) d[h][s] = fma4(a[h], b(K, s), d[h][s]);
             }
 #pragma unroll
             for (int h = 0; h < 2; h++)
@@ -379,7 +384,7 @@ __device__ inline void prot_ops(const InstDev& I, const ModelDev& m, const TileO
         for (int K = 0; K < kX; K++) {
             const d2 a = block2(10 + K / 2);
 #pragma unroll
-            for (int s = 0; s < kSets; s++) d[s] = fma4(a[K & 1], b.v[K][s], d[s]);
+            for (int s = 0; s < kSets; s++) d[s] = fma4(a[K & 1], b(K, s), d[s]);
         }
 #pragma unroll
         for (int s = 0; s < kSets; s++) put(s, 4, d[s]);
@@ -417,7 +422,7 @@ __device__ inline void prot_ops(const InstDev& I, const ModelDev& m, const TileO
                 for (int s = 0; s < kSets; s++) {
                     const double* row = tip_sh + (end[3] >> j & 1 ? I.SU + 1 : kid[j].st[s]) * kProtN + k;
 #pragma unroll
-                    for (int K = 0; K < kX; K++) kid[j].v[K][s] = row[4 * K];
+                    for (int K = 0; K < kX; K++) kid[j].set(K, s, row[4 * K]);
                 }
             }
             asm("" : "+s"(slots));   // ifs, not a switch, whose joins would copy what is being loaded
@@ -445,7 +450,7 @@ __device__ inline void prot_ops(const InstDev& I, const ModelDev& m, const TileO
         for (int j = 0; j < 2; j++) {
             const unsigned kind = kinds >> 2 * j & 3;
             const double* e = e_sh + j * kProtKid;
-            auto put = [&](int s, int X, double v) { f.v[X][s] = j == 0 ? v : f.v[X][s] * v; };
+            auto put = [&](int s, int X, double v) { f.set(X, s, j == 0 ? v : f(X, s) * v); };
             if (kind == CHILD_TIP && lut) {
 #pragma unroll
                 for (int s = 0; s < kSets; s++)
@@ -465,14 +470,14 @@ __device__ inline void prot_ops(const InstDev& I, const ModelDev& m, const TileO
         const int ahead = o + 1 < nops;
         tab += ahead * table_size;   // 2 * table_size values
         load_tables();
-        mul(inv_sh, f, [&](int s, int X, double v) { last.v[X][s] = v; });
+        mul(inv_sh, f, [&](int s, int X, double v) { last.set(X, s, v); });
         // patterns with every value below the threshold, in all categories in normal mode
         unsigned small = 0;
 #pragma unroll
         for (int s = 0; s < kSets; s++) {
             double mx = 0.0;
 #pragma unroll
-            for (int X = 0; X < kX; X++) mx = fmax(mx, fabs(last.v[X][s]));
+            for (int X = 0; X < kX; X++) mx = fmax(mx, fabs(last(X, s)));
             unsigned long long b = __builtin_amdgcn_ballot_w64(mx < Prec<double>::threshold);
             b &= b >> 32;
             b &= b >> 16;
@@ -495,7 +500,7 @@ __device__ inline void prot_ops(const InstDev& I, const ModelDev& m, const TileO
             for (int s = 0; s < kSets; s++)
                 if (small >> (16 * s + (l & 15)) & 1)
 #pragma unroll
-                    for (int X = 0; X < kX; X++) last.v[X][s] = Prec<double>::apply(last.v[X][s], 1);
+                    for (int X = 0; X < kX; X++) last.set(X, s, Prec<double>::apply(last(X, s), 1));
             sc += small >> (l & 31) & 1;
         }
         sc_last = sc;

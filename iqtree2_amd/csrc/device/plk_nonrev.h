@@ -252,7 +252,7 @@ k_nr_root(InstDev I, NrRoot R, double* __restrict__ block_sums) {
             const double* l0 = R.lut + ((size_t)s * C + c) * N;
 #pragma unroll
             for (int x = 0; x < N; x++) {
-                const double nv = (double)pn[x * Part<T, N, C>::stride];
+                const double nv = (double)pn[Part<T, N, C>::x(p, x)];
                 u0 = fma(nv, l0[x], u0);
                 if (R.derv) {
                     u1 = fma(nv, l0[ls + x], u1);
@@ -263,7 +263,7 @@ k_nr_root(InstDev I, NrRoot R, double* __restrict__ block_sums) {
             const T* pd = reinterpret_cast<const T*>(I.partial) + Part<T, N, C>::at(I, R.dad_slot, p, c);
             double dv[N];
 #pragma unroll
-            for (int y = 0; y < N; y++) dv[y] = (double)pd[y * Part<T, N, C>::stride];
+            for (int y = 0; y < N; y++) dv[y] = (double)pd[Part<T, N, C>::x(p, y)];
             const double* T0 = R.T + (size_t)c * N * N;
             const double* T1 = T0 + (size_t)C * N * N;
             const double* T2 = T1 + (size_t)C * N * N;
@@ -277,7 +277,7 @@ k_nr_root(InstDev I, NrRoot R, double* __restrict__ block_sums) {
                         v2 = fma(T2[x * N + y], dv[y], v2);
                     }
                 }
-                const double nv = (double)pn[x * Part<T, N, C>::stride];
+                const double nv = (double)pn[Part<T, N, C>::x(p, x)];
                 u0 = fma(nv, v0, u0);
                 u1 = fma(nv, v1, u1);
                 u2 = fma(nv, v2, u2);

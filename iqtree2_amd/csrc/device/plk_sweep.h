@@ -496,14 +496,14 @@ __device__ inline bool theta_first_eval(const SweepArgs& a, const SweepRes<T>& R
         const int p = tile * PB + threadIdx.x / C;
         const T* nsrc = partial + Part<T, N, C>::at(I, node.id, p, c);
 #pragma unroll
-        for (int i = 0; i < N; i++) nr[m][i] = nsrc[i * Part<T, N, C>::stride];
+        for (int i = 0; i < N; i++) nr[m][i] = nsrc[Part<T, N, C>::x(p, i)];
         scr[m] = scale[Part<T, N, C>::count_at(I, node.id, p, c)];
         if (dad.is_tip) {
             sr[m] = I.states[(size_t)dad.id * I.Ppad + p];
         } else {
             const T* dsrc = partial + Part<T, N, C>::at(I, dad.id, p, c);
 #pragma unroll
-            for (int i = 0; i < N; i++) dr[m][i] = dsrc[i * Part<T, N, C>::stride];
+            for (int i = 0; i < N; i++) dr[m][i] = dsrc[Part<T, N, C>::x(p, i)];
             scr[m] += scale[Part<T, N, C>::count_at(I, dad.id, p, c)];
         }
     }
