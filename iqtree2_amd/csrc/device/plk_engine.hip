@@ -1603,7 +1603,11 @@ plk_status launch_sweep_t(plk_context* ctx, Instance* in, SweepArgs& a, int& gri
     if (nb < 1) return fail(PLK_ERR_UNSUPPORTED, "sweep kernel does not fit a CU");
     const int PB = kThreads / C;
     const int ntiles = in->Ppad / PB;
-    const int per_cu = std::min(nb, ctx->sweep_blocks_per_cu);
+    // one workgroup a CU while that is four tiles or fewer: an exchange of half
+    // as many workgroups is shorter (444 -> 256: 3079 -> 2080 us of a sweep of
+    // 100 taxa x 30,000), which outweighs the latency that a second one hides
+    // (at seven tiles it no longer does: 1796 us against 1750, 30 taxa x 100,000)
+    const int per_cu = N == 4 && ntiles <= 4 * ctx->num_cu ? 1 : std::min(nb, ctx->sweep_blocks_per_cu);
     int grid = ctx->num_cu * per_cu;
     grid = std::max(1, std::min(grid, std::min(ntiles, 2 * kThreads)));   // the exchange polls 2 per thread
     // theta (and the per-pattern scalars) of each workgroup's tiles resident

@@ -179,7 +179,22 @@ __device__ inline bool grid_sum2(const SweepArgs& a, double v0, double v1, unsig
         if (n == 4) { s0 += x[2]; s1 += x[3]; }
     }
     if (!ok) ok_sh = 0;
-    tree_sum2(s0, s1, red_sh, res);
+    if (G <= 64) {
+        // the first wave has all the values: its sum, as tree_sum2 adds it,
+        // and one barrier in place of two (a sweep of 20 taxa x 1,000: 828
+        // -> 800 us)
+        if (threadIdx.x < 64) {
+            s0 = wave_sum(s0);
+            s1 = wave_sum(s1);
+            if (threadIdx.x == 0) {
+                res[0] = s0 + 0.0;
+                res[1] = s1 + 0.0;
+            }
+        }
+        __syncthreads();
+    } else {
+        tree_sum2(s0, s1, red_sh, res);
+    }
     if (threadIdx.x == 0) {
         // every workgroup has read exchange e-1: re-arm this workgroup's
         // slots of its buffer for exchange e+2
