@@ -760,9 +760,10 @@ template <int C> struct Mat4<double, C> {
         }
     }
     __device__ static void load_row(const Hbm<double>*, bool, int, int, double (&)[kRow]) {}
-    // a tip's product: its matrices times the tip vectors (the root leaf's: times 1, 0, 0, 0)
+    // a tip's product: its matrices times the tip vectors (the root leaf's: times 1, 0, 0, 0),
+    // 1 for the unknown state su
     __device__ static void tip(const A& a, const double (&)[kRow], const unsigned (&st)[kStates], bool root,
-                               const double* tip_sh, int lane, double (&f)[4]) {
+                               const double* tip_sh, int su, int lane, double (&f)[4]) {
         int s[4];
         if constexpr (kWords) {
 #pragma unroll
@@ -781,11 +782,14 @@ template <int C> struct Mat4<double, C> {
         if (root) {
 #pragma unroll
             for (int g = 0; g < 4; g++) b[g] = lane < 16 ? 1.0 : 0.0;
+            su = -1;
         } else {
 #pragma unroll
             for (int g = 0; g < 4; g++) b[g] = tip_sh[s[g] * 4 + (lane >> 4)];
         }
         mul(a, b, f);
+#pragma unroll
+        for (int g = 0; g < 4; g++) f[g] = s[g] == su ? 1.0 : f[g];
     }
     // pairs with every value below the threshold, as a mask
     __device__ static unsigned long long small(const double (&d)[4]) {
@@ -860,7 +864,7 @@ template <int C> struct Mat4<float, C> {
         for (int x = 0; x < 4; x++) row[x] = w[x];
     }
     __device__ static void tip(const A&, const float (&row)[kRow], const unsigned (&)[kStates], bool, const double*, int,
-                               float (&f)[4]) {
+                               int, float (&f)[4]) {
 #pragma unroll
         for (int x = 0; x < 4; x++) f[x] = row[x];
     }
@@ -1005,7 +1009,7 @@ __device__ inline void dna_ops(const InstDev& I, const ModelDev& m, const TileOp
         for (int k = 0; k < 2; k++) {
             const unsigned kind = kinds >> 2 * k & 3;
             if (kind == CHILD_TIP) {
-                M::tip(in.e[k], in.row[k], st.w[k], d.end[3] >> k & 1, tip_sh, lane, f[k]);
+                M::tip(in.e[k], in.row[k], st.w[k], d.end[3] >> k & 1, tip_sh, I.SU, lane, f[k]);
             } else if (kind == CHILD_LAST) {
                 M::mul(in.e[k], last, f[k]);
                 sc += last_sc;

@@ -456,6 +456,10 @@ __device__ inline void prot_ops(const InstDev& I, const ModelDev& m, const TileO
                 for (int s = 0; s < kSets; s++)
 #pragma unroll
                     for (int X = 0; X < kX; X++) put(s, X, e[kid[j].st[s] * kProtN + 4 * X + k]);
+            } else if (kind == CHILD_TIP) {
+                // 1 for the unknown state, as in a lookup
+                const int su = end[3] >> j & 1 ? -1 : I.SU;
+                mul(e, kid[j], [&](int s, int X, double v) { put(s, X, kid[j].st[s] == su ? 1.0 : v); });
             } else if (kind == CHILD_LAST) {
                 mul(e, last, put);
                 sc += sc_last;
