@@ -775,6 +775,7 @@ plk_status stage_ops(plk_context* ctx, Instance* in, const plk_op* ops, int nops
         in->tables = nullptr;
         in->tops = nullptr;
         const int cap = std::max(nops, 2 * in->ops_cap);
+        in->ops_cap = 0;   // until every allocation is made: a later, shorter list must not find a part of them
         st = dmalloc(ctx, in, &in->ops, sizeof(plk_op) * cap);
         if (st != PLK_OK) return st;
         st = dmalloc(ctx, in, &in->tables, (size_t)(cap + 2) * 2 * in->table_size * elem);   // dna_ops reads two steps on
