@@ -138,7 +138,7 @@ __device__ inline ModelDev on_hbm(ModelDev m) {
 template <typename T, int N, int C>
 struct Part {
     static constexpr bool kDna = N == 4, kProt = N == 20 && sizeof(T) == 8, kLanes = kDna && sizeof(T) == 8;
-    __host__ __device__ static size_t at(const InstDev& I, int slot, int p, int c) {
+    __device__ static size_t at(const InstDev& I, int slot, int p, int c) {
         if (kProt) return slot * I.slot_stride + ((size_t)(p >> 5) * C + c) * 640 + (p >> 4 & 1) * 256 + (p & 15) * 2;
         if (!kDna) return slot * I.slot_stride + (size_t)p * (N * C) + c * N;
         const int l = pair(p, c);
@@ -146,16 +146,16 @@ struct Part {
         return ((size_t)(p / (64 / C)) * I.chunk_slots + slot) * 256 + in;
     }
     // value i, from at(), where value 0 is
-    __host__ __device__ static int x(int p, int i) {
+    __device__ static int x(int p, int i) {
         if (kProt && i < 16) return (i >> 3) * 128 + (i & 3) * 32 + (i >> 2 & 1);
         if (kProt) return 512 - 255 * (p >> 4 & 1) + (i & 3) * 32;
         return kLanes ? 32 * i : i;
     }
-    __host__ __device__ static size_t count_at(const InstDev& I, int slot, int p, int c) {
+    __device__ static size_t count_at(const InstDev& I, int slot, int p, int c) {
         if (!kDna) return slot * I.scale_stride + (I.safe ? (size_t)p * C + c : (size_t)p);
         return ((size_t)(p / (64 / C)) * I.chunk_slots + slot) * 64 + pair(p, c);
     }
-    __host__ __device__ static int pair(int p, int c) { return (p % (64 / C) >> 2) * (4 * C) + 4 * c + (p & 3); }
+    __device__ static int pair(int p, int c) { return (p % (64 / C) >> 2) * (4 * C) + 4 * c + (p & 3); }
     // the thread of (p, c) writes a counter of its own
     __device__ static bool counts(const InstDev& I, int c) { return kDna || I.safe || c == 0; }
 };
@@ -1182,6 +1182,27 @@ k_traverse(InstDev I, ModelDev m, const TileOp* __restrict__ tops, int nops,
         block_sum<1>(v, reinterpret_cast<double*>(smem));
         if (threadIdx.x == 0) block_sums[blockIdx.x] = v[0];
     }
+}
+
+// Patterns p0 .. p0 + n - 1 of a slot in the order of the interface: values
+// [n][C][N], counters [n][safe ? C : 1], either may be null. Both are pinned
+// host memory, written once and in order: bound by the host link.
+template <typename T, int N, int C>
+__global__ void __launch_bounds__(kThreads)
+k_read_slot(InstDev I, int slot, int p0, int n, T* __restrict__ values, int32_t* __restrict__ counts) {
+    using L = Part<T, N, C>;
+    const T* partial = reinterpret_cast<const T*>(I.partial);
+    const typename Prec<T>::scale_t* scale = reinterpret_cast<const typename Prec<T>::scale_t*>(I.scale);
+    const size_t first = (size_t)blockIdx.x * kThreads + threadIdx.x, stride = (size_t)gridDim.x * kThreads;
+    if (values)
+        for (size_t t = first; t < (size_t)n * (N * C); t += stride) {
+            const int p = p0 + (int)(t / (N * C)), c = (int)(t / N % C), i = (int)(t % N);
+            values[t] = partial[L::at(I, slot, p, c) + L::x(p, i)];
+        }
+    const int nc = I.safe ? C : 1;
+    if (counts)
+        for (size_t t = first; t < (size_t)n * nc; t += stride)
+            counts[t] = (int32_t)scale[L::count_at(I, slot, p0 + (int)(t / nc), (int)(t % nc))];
 }
 
 // ---------------------------------------------------------------------------
