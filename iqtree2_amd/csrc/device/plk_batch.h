@@ -130,8 +130,7 @@ k_prep_batch(const BatchItem* __restrict__ items, const double* __restrict__ len
         }
         if ((n == 4 || (n == kProtN && !it.f32)) && threadIdx.x == 0) {
             TileOp* tops = hbm(const_cast<TileOp*>(it.tops));
-            if (it.f32) make_tile_op<float>(it.I, it.ops, o, it.nops, tops);
-            else make_tile_op<double>(it.I, it.ops, o, it.nops, tops);
+            make_tile_op(it.I, it.ops, o, it.nops, tops);
         }
     }
     if (blockIdx.y != 0) return;
@@ -270,7 +269,7 @@ __device__ __forceinline__ double batch_tile(const BatchItem& it, int tile, unsi
         prot_ops_tile<T, C, kBatchSub>(I, m.inv_evec, ops, it.nops, tables, it.table_size,
                                        reinterpret_cast<T*>(smem), tile * PB);
     } else {
-        dna_ops<T, C, false>(I, m, it.tops, it.nops, tables, it.table_size, tile * PB, reinterpret_cast<double*>(smem));
+        dna_ops<T, C>(I, m, it.tops, it.nops, tables, it.table_size, tile * PB, reinterpret_cast<double*>(smem));
     }
     double* root_sh = reinterpret_cast<double*>(smem);
     const plk_end node = it.node, dad = it.dad;

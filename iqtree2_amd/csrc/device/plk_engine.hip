@@ -89,7 +89,6 @@ struct Instance {
     size_t elem = 8;            // bytes of one stored value
     size_t scale_elem = 2;      // bytes of one scale counter
     int table_size = 0;         // elements per (op, child) table
-    int chunk_slots = 0;        // slots of a chunk (Part)
     int sweep_table_size = 0;   // elements per child table in the sweep's LDS layout
     size_t bytes = 0;           // HBM held
     // device buffers
@@ -163,9 +162,8 @@ struct Instance {
 
 size_t alloc_class(size_t bytes);
 
-// slots the arrays hold: 4 states an odd number; and counters of a pattern (Part)
-int stored_slots(const plk_instance_desc* d) { return d->nstates == 4 ? d->nslots | 1 : d->nslots; }
-int stored_counts(const plk_instance_desc* d) { return d->safe_numeric || d->nstates == 4 ? d->ncat : 1; }
+// scale counters of a pattern in a slot
+int stored_counts(const plk_instance_desc* d) { return d->safe_numeric ? d->ncat : 1; }
 
 // op lists that the traversal reads as TileOps
 bool has_tile_ops(const plk_instance_desc* d) {
@@ -194,8 +192,8 @@ size_t footprint_of(const plk_instance_desc* d, int Ppad) {
         (size_t)d->ntaxa * Ppad,                                  // states
         (size_t)Ppad * 8, (size_t)Ppad * 8,                       // freq, invar
         (n + 2 * n * n + (SU + 1) * n + 2 * (size_t)d->ncat) * 8, // model
-        (size_t)stored_slots(d) * Ppad * block * elem,            // partials
-        (size_t)stored_slots(d) * Ppad * ncnt * scale_elem,       // scale counters
+        (size_t)d->nslots * Ppad * block * elem,            // partials
+        (size_t)d->nslots * Ppad * ncnt * scale_elem,       // scale counters
         (size_t)Ppad * block * elem,                              // theta
         (size_t)Ppad * 8, (size_t)Ppad * 8,                       // buffer_scale, ptn_lh
         (size_t)(Ppad / (kThreads / 8) + 1) * 3 * 8,              // block sums
@@ -442,8 +440,9 @@ InstDev inst_dev(const Instance* in) {
     I.buffer_scale = in->buffer_scale;
     I.ptn_lh = in->ptn_lh;
     I.slot_stride = (size_t)in->Ppad * in->block;
-    I.scale_stride = (size_t)in->Ppad * (in->d.safe_numeric ? in->d.ncat : 1);
-    I.chunk_slots = in->chunk_slots;
+    I.scale_stride = (size_t)in->Ppad * stored_counts(&in->d);
+    I.slot_units = (uint32_t)(I.slot_stride * in->elem >> 8);
+    I.scale_units = (uint32_t)(I.scale_stride * in->scale_elem >> 8);
     I.nasc = in->nasc;
     I.asc = in->nasc > kAscMax ? in->asc_vals : in->red_out + 8;
     return I;
@@ -532,8 +531,7 @@ plk_status launch_traverse_t(plk_context* ctx, Instance* in, int nops, int mode,
                            nops, reinterpret_cast<const T*>(in->tables), in->table_size, mode, node, dad,
                            in->root_tab, in->block_sums);
     };
-    if (dna_far(in->chunk_slots, sizeof(T))) go(k_traverse<T, N, C, true>);
-    else go(k_traverse<T, N, C, false>);
+    go(k_traverse<T, N, C>);
     HIP_TRY(hipGetLastError());
     if (pe >= 0) {
         const double P = in->d.npatterns, s = (double)in->elem, blk = (double)in->block;
@@ -1124,7 +1122,6 @@ plk_status plk_instance_create(plk_context* ctx, const plk_instance_desc* d, int
     in->d = *d;
     in->Ppad = Ppad;
     in->block = (size_t)d->nstates * d->ncat;
-    in->chunk_slots = stored_slots(d);
     in->elem = d->precision == PLK_PREC_F32 ? 4 : 8;
     in->scale_elem = d->precision == PLK_PREC_F32 ? 4 : 2;
     in->sweep_table_size = (int)std::max(in->block * d->nstates, (size_t)(d->state_unknown + 1) * in->block);
@@ -1143,8 +1140,8 @@ plk_status plk_instance_create(plk_context* ctx, const plk_instance_desc* d, int
     A(&in->freq, (size_t)Ppad * 8);
     A(&in->invar, (size_t)Ppad * 8);
     A(&in->model, model_doubles * 8);
-    A(&in->partial, (size_t)in->chunk_slots * Ppad * in->block * in->elem);
-    A(&in->scale, (size_t)in->chunk_slots * Ppad * ncnt * in->scale_elem);
+    A(&in->partial, (size_t)d->nslots * Ppad * in->block * in->elem);
+    A(&in->scale, (size_t)d->nslots * Ppad * ncnt * in->scale_elem);
     A(&in->theta, (size_t)Ppad * in->block * in->elem);
     A(&in->buffer_scale, (size_t)Ppad * 8);
     A(&in->ptn_lh, (size_t)Ppad * 8);
@@ -1156,7 +1153,7 @@ plk_status plk_instance_create(plk_context* ctx, const plk_instance_desc* d, int
         if (hipMemsetAsync(in->states, d->state_unknown, (size_t)d->ntaxa * Ppad, ctx->stream) != hipSuccess ||
             hipMemsetAsync(in->freq, 0, (size_t)Ppad * 8, ctx->stream) != hipSuccess ||
             hipMemsetAsync(in->invar, 0, (size_t)Ppad * 8, ctx->stream) != hipSuccess ||
-            hipMemsetAsync(in->scale, 0, (size_t)in->chunk_slots * Ppad * ncnt * in->scale_elem, ctx->stream) != hipSuccess ||
+            hipMemsetAsync(in->scale, 0, (size_t)d->nslots * Ppad * ncnt * in->scale_elem, ctx->stream) != hipSuccess ||
             hipStreamSynchronize(ctx->stream) != hipSuccess)
             st = fail(PLK_ERR_DEVICE, "initialising instance buffers failed");
     }
@@ -2022,7 +2019,7 @@ plk_status plk_batch_evaluate(plk_context* ctx, const plk_batch_item* items, con
     bool nonfinite = false;
     for (int i = 0; i < nitems; i++) {
         const Instance* in = ins[i];
-        if (in->d.ncat == 4 && in->nasc == 0 && !in->nonrev && !(in->d.nstates == 4 && dna_far(in->chunk_slots, in->elem)) &&
+        if (in->d.ncat == 4 && in->nasc == 0 && !in->nonrev &&
             (in->d.nstates == 4 || in->d.nstates == 20 || in->d.nstates == kCodonN)) {
             fused.push_back(items[i]);
             fused_ins.push_back(ins[i]);

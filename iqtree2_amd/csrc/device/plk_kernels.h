@@ -2,16 +2,17 @@
 //
 // Layout in HBM (one instance):
 //   partial[slot][p][c][x]   T (double or float), pattern-major, eigen basis;
-//                            4 states: in chunks of 64 pairs, Part below
+//                            4 states, and 20 in double storage: as Part says
 //   scale[slot][p]           uint16 (FP64 form) / int32 exponent (FP32 form),
-//                            [slot][p][c] in safe mode; 4 states as Part says
+//                            [slot][p][c] in safe mode
 //   theta[p][c][x]           T; buffer_scale[p] double
 //   states[taxon][p]         uint8
 // Thread mapping: one thread per (pattern, category); the C threads of a
 // pattern are adjacent lanes of one wavefront, so cross-category reductions are
-// lane shuffles. A workgroup owns a tile of 256/C patterns
-// and walks the whole post-order op list for that tile: patterns are
-// independent, so no synchronisation crosses workgroups.
+// lane shuffles. The traversals of 4 states (dna_ops) and of 20 in double
+// storage (prot_ops) map lanes as their matrix products do. A workgroup owns a
+// tile of 256/C patterns and walks the whole post-order op list for that tile:
+// patterns are independent, so no synchronisation crosses workgroups.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -83,7 +84,7 @@ struct InstDev {
     double* ptn_lh;          // [Ppad]
     size_t slot_stride;      // Ppad*block
     size_t scale_stride;     // Ppad*(safe?C:1)
-    int chunk_slots;         // 4 states: slots of a chunk (Part)
+    uint32_t slot_units, scale_units;   // the same in 256 bytes (whole: Ppad is a multiple of 256)
     // +ASC (Lewis): the last nasc of the P patterns are the unobserved
     // constant patterns; pattern k's lh goes to asc[4k], and a derivative
     // evaluation adds lh as the derivative sum counts it, d1 and d2 at 4k+1..3
@@ -116,19 +117,22 @@ __device__ inline ModelDev on_hbm(ModelDev m) {
 }
 
 // Where slot s keeps value x of (pattern p, category c), element
-// at(I, s, p, c) + x(p, x), and its counter, element count_at(I, s, p, c)
-// ([slot][p], safe mode [slot][p][c]; 4 states one per pair in both modes, so
-// that a wavefront writes whole lines).
+// at(I, s, p, c) + x(p, x), and its counter, element count_at(I, s, p, c):
+// [slot][p], safe mode [slot][p][c]. Values are [slot][p][c][x], but
 // 4 states: 64 (pattern, category) pairs, those of 64 / C adjacent patterns,
-// make a chunk, and a chunk keeps all its slots together, so that the
-// wavefront that walks a tree for it (dna_ops) stays in one stretch of memory
-// and addresses it by 32-bit offsets. A chunk has an odd number of slots:
-// wavefronts that write the same slot at a time then spread over the memory
-// channels (200 taxa x 100,000 sites, even: 1,042 us, odd: 1,031). In a chunk's slot, four patterns' pairs
-// of a category are adjacent: pair (p / 4, c, p % 4), and pair l's values are
+// make a chunk of 256 values, and in it four patterns' pairs of a category are
+// adjacent: pair l = (p / 4, c, p % 4), whose values are
 //   float    at 4l + x
 //   double   at [g / 2][x][j][g % 2] of pair l = j + 16g (j < 16): a lane's
 //            matrix operands, sixteen bytes at a time
+// A slot is one stretch of memory, since a sweep reads a slot of all patterns
+// at a time: with all slots of a chunk together a pass over the branches of
+// 200 taxa x 100,000 sites took 17.2 ms (so: 17.0; float 14.9 and 14.4), and
+// the float traversal of 100 x 100,000 took 367 us (so: 357; double 437 both).
+// A thread of its own pair reads four values of eight bytes. With two values
+// of a pair side by side, and lanes that exchange rows around each load and
+// store of dna_ops, the pass took 16.65 ms and an NNI round of it 120 ms (so:
+// 123), but one branch's Newton 148 us (144) and small batches 3 to 5% more.
 // 20 states in double storage: 32 patterns of a category make a block of 640
 // values, the operand registers X = x / 4 of a wavefront's two sixteens S, two
 // side by side: [(S0, X0 X1), (S0, X2 X3), the same of S1, (X4, S0 S1)]
@@ -138,12 +142,13 @@ __device__ inline ModelDev on_hbm(ModelDev m) {
 template <typename T, int N, int C>
 struct Part {
     static constexpr bool kDna = N == 4, kProt = N == 20 && sizeof(T) == 8, kLanes = kDna && sizeof(T) == 8;
-    __device__ static size_t at(const InstDev& I, int slot, int p, int c) {
+    // (unsigned, so that a thread's place within its tile is worked out once)
+    __device__ static size_t at(const InstDev& I, int slot, uint32_t p, uint32_t c) {
         if (kProt) return slot * I.slot_stride + ((size_t)(p >> 5) * C + c) * 640 + (p >> 4 & 1) * 256 + (p & 15) * 2;
         if (!kDna) return slot * I.slot_stride + (size_t)p * (N * C) + c * N;
-        const int l = pair(p, c);
-        const int in = kLanes ? (l >> 5) * 128 + (l & 15) * 2 + (l >> 4 & 1) : l * 4;
-        return ((size_t)(p / (64 / C)) * I.chunk_slots + slot) * 256 + in;
+        const uint32_t l = (p % (64 / C) >> 2) * (4 * C) + 4 * c + (p & 3);
+        return (size_t)((uint32_t)slot * I.slot_units) * (256 / sizeof(T)) + (size_t)(p / (64 / C)) * 256 +
+               (kLanes ? (l >> 5) * 128 + (l & 15) * 2 + (l >> 4 & 1) : l * 4);
     }
     // value i, from at(), where value 0 is
     __device__ static int x(int p, int i) {
@@ -151,13 +156,10 @@ struct Part {
         if (kProt) return 512 - 255 * (p >> 4 & 1) + (i & 3) * 32;
         return kLanes ? 32 * i : i;
     }
-    __device__ static size_t count_at(const InstDev& I, int slot, int p, int c) {
+    __device__ static size_t count_at(const InstDev& I, int slot, uint32_t p, uint32_t c) {
         if (!kDna) return slot * I.scale_stride + (I.safe ? (size_t)p * C + c : (size_t)p);
-        return ((size_t)(p / (64 / C)) * I.chunk_slots + slot) * 64 + pair(p, c);
+        return (size_t)((uint32_t)slot * I.scale_units) * (256 / sizeof(typename Prec<T>::scale_t)) + (I.safe ? p * C + c : p);
     }
-    __device__ static int pair(int p, int c) { return (p % (64 / C) >> 2) * (4 * C) + 4 * c + (p & 3); }
-    // the thread of (p, c) writes a counter of its own
-    __device__ static bool counts(const InstDev& I, int c) { return kDna || I.safe || c == 0; }
 };
 
 // Elements of one (op, child) table for 4 states. Double storage: a child's
@@ -235,33 +237,23 @@ enum BufferMode { BUF_DERV = 0, BUF_LNL = 1 };
 // each made when its part of the step is due.
 struct alignas(64) TileOp {
     uint64_t tip[2];      // a tip child's row of states (others: taxon 0's)
-    uint32_t v[2], sc[2]; // a slot child's values and counters, kNoSlot for one that comes from elsewhere
-    uint32_t dst, dsc;    // the dad's; offsets in bytes from the chunk's slot 0 (far instances and 20 states: slots)
+    uint32_t v[2], sc[2]; // where a slot child's values and counters begin, kNoSlot for one that comes from elsewhere
+    uint32_t dst, dsc;    // the dad's; in units of 256 bytes from slot 0, so that 32 bits reach 1 TB (20 states: slots)
     uint32_t kind;        // of child k in bits 2k and 2k + 1, below
     uint32_t root;        // bit k: child k is the root leaf (state-basis models)
 };
 // a slot in memory, the dad of the step before (in registers), the dad of the
 // step before that, a tip
 enum TileChild { CHILD_SLOT = 0, CHILD_LAST = 1, CHILD_LAST2 = 2, CHILD_TIP = 3 };
-constexpr uint32_t kNoSlot = 0xFFFFF800u;    // past the end of a chunk's buffer
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 constexpr int kTileAhead = 6;                // steps that dna_ops looks ahead: copies of the last TileOp
 
-// bytes of a chunk's slot: values, counters
-template <typename T> constexpr uint32_t kChunkValues = 256 * sizeof(T);
-template <typename T> constexpr uint32_t kChunkCounts = 64 * sizeof(typename Prec<T>::scale_t);
-// a chunk of more slots than 32-bit offsets reach (two million in double storage)
-__host__ __device__ inline bool dna_far(int chunk_slots, size_t elem) {
-    return (uint64_t)chunk_slots * 256 * elem > kNoSlot;
-}
-
 // steps nops .. nops + kTileAhead - 1 repeat the last
-template <typename T>
 __device__ inline void make_tile_op(const InstDev& I, const plk_op* __restrict__ ops, int o, int nops, TileOp* tops,
                                     unsigned root = 0) {
     const plk_op op = ops[o];
     const int last = o > 0 ? ops[o - 1].dad_slot : -1, last2 = o > 1 ? ops[o - 2].dad_slot : -1;
-    const bool far = I.n != 4 || dna_far(I.chunk_slots, sizeof(T));
-    const uint32_t nv = far ? 1 : kChunkValues<T>, nc = far ? 1 : kChunkCounts<T>;
+    const uint32_t nv = I.n != 4 ? 1 : I.slot_units, nc = I.n != 4 ? 1 : I.scale_units;
     TileOp t;
     t.kind = 0;
     for (int k = 0; k < 2; k++) {
@@ -296,7 +288,7 @@ k_prep_ops(const plk_op* __restrict__ ops, int nops, ModelDev m, int n, int C, i
     extern __shared__ double sh[];
     const int o = blockIdx.x >> 1, k = blockIdx.x & 1, c = blockIdx.y;
     if (o >= nops) return;
-    if (tops && k == 0 && c == 0 && threadIdx.x == 0) make_tile_op<T>(I, ops, o, nops, tops);
+    if (tops && k == 0 && c == 0 && threadIdx.x == 0) make_tile_op(I, ops, o, nops, tops);
     const plk_child ch = ops[o].child[k];
     double* ex = sh;
     for (int i = threadIdx.x; i < n; i += blockDim.x) ex[i] = exp(m.eval[i] * (m.rates[c] * ch.length));
@@ -632,7 +624,7 @@ __device__ inline void op_finish(const InstDev& I, const T* inv_sh, const T* tL,
     T* dst = partial + Part<T, N, C>::at(I, dad_slot, p, c);
 #pragma unroll
     for (int i = 0; i < N; i++) dst[Part<T, N, C>::x(p, i)] = dadv[i];
-    if (Part<T, N, C>::counts(I, c)) scale[Part<T, N, C>::count_at(I, dad_slot, p, c)] = (ST)sc;
+    if (safe || c == 0) scale[Part<T, N, C>::count_at(I, dad_slot, p, c)] = (ST)sc;
 }
 
 template <typename T, int N, int C>
@@ -664,13 +656,11 @@ __device__ inline void op_apply(const InstDev& I, const T* inv_sh, const T* tL, 
 //   - what a step reads is loaded two steps ahead. Loads and stores share one
 //     in-order counter, so a wait for a load is one for all before it, but not
 //     for the stores of the two steps since;
-//   - a step makes few accesses: both children's matrices in one, and the tips'
-//     states through the scalar cache. Of 200 taxa x 100,000 sites' 858 us with
-//     13 vector accesses a step, 430 went into the stores, at the rate of a
-//     fill, 165 into children (most of them not needed, read past the end of
-//     a buffer), 110 into states and 108 into matrices, one after the other.
-// Measured, whole kernel, 198 steps: 1,000 patterns 415 -> 125 us, 99,390
-// patterns 1,153 -> 711 us in double (5.1 GB algorithmic, 2.6 GB written).
+//   - a step makes few accesses: both children's matrices in one, the tips'
+//     states through the scalar cache, and slots only of children that are read.
+// Measured, whole kernel, 198 steps: 1,000 patterns 136 us, 100,000
+// 695 us in double (2.6 GB written), the kernel of a thread a pair,
+// with tables in LDS, 415 and 1,153.
 typedef unsigned tile_u4 __attribute__((ext_vector_type(4)));
 using Buffer = __amdgpu_buffer_rsrc_t;
 
@@ -893,8 +883,8 @@ template <int C> struct Mat4<float, C> {
 __host__ __device__ inline size_t dna_ops_smem(int SU) { return (size_t)(SU + 1) * 4 * sizeof(double); }
 
 // p_first: the workgroup's first of 256 / C patterns (uniform). tip_sh:
-// dna_ops_smem(SU). kFar: instances of dna_far, a buffer of its own for each slot.
-template <typename T, int C, bool kFar>
+// dna_ops_smem(SU).
+template <typename T, int C>
 __device__ inline void dna_ops(const InstDev& I, const ModelDev& m, const TileOp* tops, int nops, const T* tables_g,
                                int table_size, int p_first, double* tip_sh) {
     using ST = typename Prec<T>::scale_t;
@@ -910,17 +900,14 @@ __device__ inline void dna_ops(const InstDev& I, const ModelDev& m, const TileOp
     const int q = Pr::pattern(lane);
     const bool no_invar = I.invar[p0 + q] == 0.0;
     const typename M::A inv = M::load_same(m.inv_evec, lane);
-    // the chunk's values and counters, and this lane's places in a slot of them
-    const size_t chunk = (size_t)(p0 / Pr::kPatterns) * I.chunk_slots;
-    constexpr uint32_t nv = kChunkValues<T>, nc = kChunkCounts<T>;
-    const uint64_t vbase = (uint64_t)I.partial + chunk * nv, cbase = (uint64_t)I.scale + chunk * nc;
-    const Buffer values_all = buffer_of(vbase, I.chunk_slots * nv), counts_all = buffer_of(cbase, I.chunk_slots * nc);
-    // the buffer that holds a slot, and where in it the slot begins
-    auto part = [](Buffer all, uint64_t base, uint32_t slot, uint32_t bytes) {
-        return kFar ? buffer_of(base + (uint64_t)slot * bytes, slot == kNoSlot ? 0 : bytes) : all;
-    };
-    auto from = [](uint32_t slot) { return kFar ? 0u : slot; };
-    const uint32_t vat = lane * 16, sat = lane * sizeof(ST);
+    // the wavefront's part of a slot: its values and counters, and this lane's places in them
+    constexpr uint32_t nv = 256 * sizeof(T);
+    const uint32_t nc = (I.safe ? 64 : Pr::kPatterns) * sizeof(ST);
+    const uint64_t vbase = (uint64_t)I.partial + (uint64_t)(p0 / Pr::kPatterns) * nv;
+    const uint64_t cbase = (uint64_t)I.scale + (uint64_t)(p0 / Pr::kPatterns) * nc;
+    auto part = [](uint64_t base, uint32_t slot, uint32_t bytes) { return buffer_of(base + ((uint64_t)slot << 8), bytes); };
+    const uint32_t vat = lane * 16, sat = (I.safe ? q * C + Pr::cat(lane) : q) * sizeof(ST);
+    const bool counting = I.safe || Pr::cat(lane) == 0;   // normal mode: a counter a pattern
 
     struct Kids {
         T v[2][4];                       // a slot's values
@@ -964,13 +951,13 @@ __device__ inline void dna_ops(const InstDev& I, const ModelDev& m, const TileOp
             M::load_row(tab + k * table_size, (kind >> 2 * k & 3) == CHILD_TIP, st.w[k][0], lane, in.row[k]);
         tab += 2 * table_size;
     };
-    // past the end of the buffers (kNoSlot) for a child that is no slot
+    // zeros (buffers of no bytes) for a child that is no slot
     auto load_slot = [&](const tile_u4 kids, int k, Kids& in) {
-        M::load_slot(part(values_all, vbase, kids[k], nv), vat + from(kids[k]), in.v[k]);
-        const Buffer counts = part(counts_all, cbase, kids[2 + k], nc);
-        const uint32_t at = sat + from(kids[2 + k]);
-        if (sizeof(ST) == 2) in.sc[k] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(counts, at, 0, 0);
-        else in.sc[k] = (int)__builtin_amdgcn_raw_buffer_load_b32(counts, at, 0, 0);
+        const bool slot = kids[k] != kNoSlot;
+        M::load_slot(part(vbase, kids[k], slot ? nv : 0), vat, in.v[k]);
+        const Buffer counts = part(cbase, kids[2 + k], slot ? nc : 0);
+        if (sizeof(ST) == 2) in.sc[k] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(counts, sat, 0, 0);
+        else in.sc[k] = (int)__builtin_amdgcn_raw_buffer_load_b32(counts, sat, 0, 0);
     };
 
     // even and odd steps have their own registers, since a copy would wait for
@@ -1043,11 +1030,12 @@ __device__ inline void dna_ops(const InstDev& I, const ModelDev& m, const TileOp
         for (int k = 0; k < 2; k++)
             if ((d.kids_end[2] >> 2 * k & 3) == CHILD_SLOT) load_slot(d.kids, k, in);
         load_states(d.tips, kTipsAhead ? CHILD_TIP | CHILD_TIP << 2 : d.kids_end[2], st);
-        M::store_slot(part(values_all, vbase, d.end[0], nv), vat + from(d.end[0]), dad);
-        const Buffer counts = part(counts_all, cbase, d.end[1], nc);
-        const uint32_t at = sat + from(d.end[1]);
-        if (sizeof(ST) == 2) __builtin_amdgcn_raw_buffer_store_b16((unsigned short)sc, counts, at, 0, 0);
-        else __builtin_amdgcn_raw_buffer_store_b32(sc, counts, at, 0, 0);
+        M::store_slot(part(vbase, d.end[0], nv), vat, dad);
+        if (counting) {
+            const Buffer counts = part(cbase, d.end[1], nc);
+            if (sizeof(ST) == 2) __builtin_amdgcn_raw_buffer_store_b16((unsigned short)sc, counts, sat, 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b32(sc, counts, sat, 0, 0);
+        }
         d = desc(o + 2);
         if constexpr (kTipsAhead) d.tips = load_u4(tp + (uint64_t)(o + 6) * sizeof(TileOp));
     };
@@ -1112,7 +1100,7 @@ __device__ inline void theta_apply(const InstDev& I, plk_end node, plk_end dad, 
 // Fused post-order traversal over the op list followed, per mode, by the
 // branch lnL (computeLikelihoodBranchSIMD 2753-3104) or the theta buffer of
 // the branch (node, dad).
-template <typename T, int N, int C, bool kFar>
+template <typename T, int N, int C>
 __global__ void __launch_bounds__(kThreads, 4)
 k_traverse(InstDev I, ModelDev m, const TileOp* __restrict__ tops, int nops,
            const T* __restrict__ tables, int table_size, int mode, plk_end node, plk_end dad,
@@ -1125,7 +1113,7 @@ k_traverse(InstDev I, ModelDev m, const TileOp* __restrict__ tops, int nops,
     const bool live = p < I.Ppad;                            // every thread: PB divides Ppad
 
     static_assert(N == 4, "20 and 61 states have their own traversal kernels");
-    dna_ops<T, C, kFar>(I, m, tops, nops, tables, table_size, blockIdx.x * PB, reinterpret_cast<double*>(smem));
+    dna_ops<T, C>(I, m, tops, nops, tables, table_size, blockIdx.x * PB, reinterpret_cast<double*>(smem));
 
     if (mode == MODE_PARTIALS) return;
 

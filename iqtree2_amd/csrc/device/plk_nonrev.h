@@ -69,7 +69,7 @@ k_nr_prep_ops(const plk_op* __restrict__ ops, const uint8_t* __restrict__ flags,
     const int o = blockIdx.x >> 1, k = blockIdx.x & 1, c = blockIdx.y;
     if (o >= nops) return;
     if (tops && k == 0 && c == 0 && threadIdx.x == 0)
-        make_tile_op<T>(I, ops, o, nops, tops,
+        make_tile_op(I, ops, o, nops, tops,
                         (flags[2 * o] & kNrRootLeaf ? 1 : 0) | (flags[2 * o + 1] & kNrRootLeaf ? 2 : 0));
     const int n = D.n, C = D.C, m = D.mix[c];
     const plk_child ch = ops[o].child[k];
