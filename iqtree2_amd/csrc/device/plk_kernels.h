@@ -778,8 +778,12 @@ template <int C> struct Mat4<double, C> {
             for (int g = 0; g < 4; g++) b[g] = tip_sh[s[g] * 4 + (lane >> 4)];
         }
         mul(a, b, f);
+        unsigned long long any = 0;
 #pragma unroll
-        for (int g = 0; g < 4; g++) f[g] = s[g] == su ? 1.0 : f[g];
+        for (int g = 0; g < 4; g++) any |= __builtin_amdgcn_ballot_w64(s[g] == su);
+        if (any)
+#pragma unroll
+            for (int g = 0; g < 4; g++) f[g] = s[g] == su ? 1.0 : f[g];
     }
     // pairs with every value below the threshold, as a mask
     __device__ static unsigned long long small(const double (&d)[4]) {
