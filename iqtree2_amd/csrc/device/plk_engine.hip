@@ -230,7 +230,7 @@ struct ProfRec {
 struct plk_context {
     int device = 0;
     int num_cu = 0;
-    int sweep_blocks_per_cu = 2;
+    int sweep_blocks_per_cu = 0;        // workgroups of a sweep per CU; 0: by the number of tiles
     bool sweep_lds = true;              // theta resident in LDS during sweeps when it fits
     int lds_per_cu = 0;                 // bytes of LDS per CU
     int mfma_sub = 1;                   // 16-pattern sub-tiles per protein traversal workgroup
@@ -1575,11 +1575,15 @@ plk_status launch_sweep_t(plk_context* ctx, Instance* in, SweepArgs& a, int& gri
     if (nb < 1) return fail(PLK_ERR_UNSUPPORTED, "sweep kernel does not fit a CU");
     const int PB = kThreads / C;
     const int ntiles = in->Ppad / PB;
-    // one workgroup a CU while that is four tiles or fewer: an exchange of half
-    // as many workgroups is shorter (444 -> 256: 3079 -> 2080 us of a sweep of
-    // 100 taxa x 30,000), which outweighs the latency that a second one hides
-    // (at seven tiles it no longer does: 1796 us against 1750, 30 taxa x 100,000)
-    const int per_cu = N == 4 && ntiles <= 4 * ctx->num_cu ? 1 : std::min(nb, ctx->sweep_blocks_per_cu);
+    // 4 states, one workgroup a CU while that is four tiles or fewer: an
+    // exchange of half as many workgroups is shorter, which outweighs the
+    // latency that a second one hides. A pass over 20 taxa, one against two a
+    // CU, at 1.6, 2.5 and 3.7 tiles a CU: double, 4 categories 922, 1030 and
+    // 1095 us against 995, 1080 and 1120; float 854, 945 and 975 against 958,
+    // 994 and 1026; 1, 2 and 8 categories alike, 2 to 12%. At 4.5 and 5.2 tiles
+    // they are the same within 1%, at seven 1796 against 1750 (30 taxa).
+    const bool lone = N == 4 && ctx->sweep_blocks_per_cu == 0 && ntiles <= 4 * ctx->num_cu;
+    const int per_cu = lone ? 1 : std::min(nb, ctx->sweep_blocks_per_cu > 0 ? ctx->sweep_blocks_per_cu : 2);
     int grid = ctx->num_cu * per_cu;
     grid = std::max(1, std::min(grid, std::min(ntiles, 2 * kThreads)));   // the exchange polls 2 per thread
     // theta (and the per-pattern scalars) of each workgroup's tiles resident
@@ -1599,8 +1603,10 @@ plk_status launch_sweep_t(plk_context* ctx, Instance* in, SweepArgs& a, int& gri
     a.lds_tiles = lds_tiles;
     // exactly per_cu workgroups on every CU: with room for one more, the
     // dispatcher may stack three on some CUs and leave others with one, and
-    // every grid-wide exchange waits for the slowest CU
-    if (ctx->lds_per_cu > 0) {
+    // every grid-wide exchange waits for the slowest CU. (No more workgroups
+    // than CUs spread by themselves: padded, the passes above took the same
+    // within 1%.)
+    if (!lone && ctx->lds_per_cu > 0) {
         const int pad = ctx->lds_per_cu / (per_cu + 1) + 256;
         int nbp = 0;
         if (pad > smem && pad <= kLdsMax &&
