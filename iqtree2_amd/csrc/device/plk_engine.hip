@@ -406,15 +406,23 @@ void prof_end(plk_context* ctx, int idx, int kind, double bytes, double flops) {
     ctx->prof_recs.push_back(ProfRec{kind, bytes, flops, idx});
 }
 
-// algorithmic bytes / flops per pattern of one traversal step: child partials
-// read once, the parent written once, one state byte per tip child, scale
-// counters read and written
-void op_cost(const Instance* in, const plk_op& op, double& bytes, double& flops) {
+// algorithmic bytes / flops per pattern of step o of a traversal: child
+// partials read once, the parent written once, one state byte per tip child,
+// scale counters read and written. The traversals by TileOps keep the last
+// dad (4 states: the last two) in registers and don't read it as a child.
+void op_cost(const Instance* in, const plk_op* ops, int o, double& bytes, double& flops) {
+    const plk_op& op = ops[o];
+    const int kept = !has_tile_ops(&in->d) ? 0 : in->d.nstates == 4 ? 2 : 1;
     const double s = (double)in->elem, n = in->d.nstates, C = in->d.ncat;
-    int k_int = 0, k_tip = 0;
-    for (int k = 0; k < op.nchildren; k++) (op.child[k].is_tip ? k_tip : k_int)++;
+    int k_int = 0, k_tip = 0, k_read = 0;
+    for (int k = 0; k < op.nchildren; k++) {
+        (op.child[k].is_tip ? k_tip : k_int)++;
+        bool read = !op.child[k].is_tip;
+        for (int a = 1; a <= std::min(kept, o); a++) read = read && op.child[k].id != ops[o - a].dad_slot;
+        k_read += read;
+    }
     const double ncnt = in->d.safe_numeric ? C : 1;
-    bytes = C * n * s * (k_int + 1) + k_tip + in->scale_elem * ncnt * (k_int + 1);
+    bytes = C * n * s * (k_read + 1) + k_tip + in->scale_elem * ncnt * (k_read + 1);
     flops = C * (2.0 * n * n * k_int + n * (k_int + k_tip - 1) + 2.0 * n * n);
 }
 
@@ -776,7 +784,7 @@ plk_status stage_ops(plk_context* ctx, Instance* in, const plk_op* ops, int nops
     in->staged_bytes = in->staged_flops = 0.0;
     for (int o = 0; o < nops; o++) {
         double b, f;
-        op_cost(in, ops[o], b, f);
+        op_cost(in, ops, o, b, f);
         in->staged_bytes += b;
         in->staged_flops += f;
     }
@@ -1831,7 +1839,7 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
         double ob = 0.0, of = 0.0;
         for (int o = 0; o < items[i].nops; o++) {
             double bb, ff;
-            op_cost(in, items[i].ops[o], bb, ff);
+            op_cost(in, items[i].ops, o, bb, ff);
             ob += bb;
             of += ff;
         }
@@ -2331,7 +2339,7 @@ plk_status plk_optimize_sweep_ex(plk_context* ctx, int id, const plk_sweep_op* o
             tmp.nchildren = 2;
             for (int k = 0; k < 2; k++) tmp.child[k].is_tip = ops[o].child[k].is_tip;
             double b, f;
-            op_cost(in, tmp, b, f);
+            op_cost(in, &tmp, 0, b, f);
             bytes += b;
             flops += f;
         }
