@@ -1,7 +1,8 @@
 """The 20-state traversal in double storage: op lists in every order a caller
 may give, pattern counts around a wavefront's two sixteens, every category
-count, both counter modes, and alphabets whose tip lookups do and do not fit
-the staged tables. Counters bit-exact and values to 1e-10 of the pattern's
+count, both counter modes, rescaling beside patterns that have a +I mass and
+are never rescaled, and alphabets whose tip lookups do and do not fit the staged
+tables. Counters bit-exact and values to 1e-10 of the pattern's
 largest against the oracle: a value is a chain of at most a few hundred
 roundings of 1.1e-16, times the twenty terms of its sums."""
 import numpy as np
@@ -50,6 +51,35 @@ def test_orders_and_edges(ctx, ncat, safe, npat, taxa, unknown):
                 assert abs(lg - lo) <= 1e-9 * abs(lo)
                 np.testing.assert_allclose(pg, po, rtol=0, atol=1e-9)
                 compare_partials(inst, orc, ops)
+    finally:
+        tree.close()
+        inst.close()
+
+
+@pytest.mark.parametrize("ncat", [1, 2, 4, 8])
+@pytest.mark.parametrize("safe", [False, True])
+def test_rescaling_beside_invariable_sites(ctx, ncat, safe):
+    print(f"ncat={ncat} safe={safe}", flush=True)
+    w = ia.Workload(seq_type=ia.PROTEIN, ntaxa=120, nsite=80, ncat=ncat, mean_len=1.0, alpha=1.0, seed=78)
+    P = min(70, w.npatterns)
+    massed = np.arange(P) % 3 == 1
+    m = w.model_arrays()
+    inst = ia.Instance(ctx, 120, 20, ncat, P, 120, w.state_unknown, safe_numeric=safe)
+    orc = OracleTree(120, 20, ncat, P, 120, w.state_unknown, safe, 2)
+    for x in (inst, orc):
+        x.set_patterns(np.ascontiguousarray(w.get("states")[:, :P]), np.ones(P), 0.01 * massed)
+        x.set_model(m["eval"], m["evec"], m["inv_evec"], m["tip"], m["rates"], m["props"])
+    tree = ia.PhyloTree(None, w)
+    try:
+        ops, node, dad = tree.plan_full(*tree.branches()[30])
+        lg, pg = inst.likelihood_branch(ops, node, dad, 0.1, want_pattern_lh=True)
+        lo, po = orc.likelihood_branch(ops, node, dad, 0.1, want_pattern_lh=True)
+        assert abs(lg - lo) <= 1e-9 * abs(lo)
+        np.testing.assert_allclose(pg, po, rtol=0, atol=1e-9)
+        compare_partials(inst, orc, ops)
+        counts = [inst.read_partial(int(op["dad_slot"]))[1] for op in ops]
+        assert not any(c[massed].any() for c in counts)
+        assert max(int(c.max()) for c in counts) > 0
     finally:
         tree.close()
         inst.close()
