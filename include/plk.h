@@ -17,9 +17,10 @@
  *   tip_eigen   [SU+1][n]             U^-1 * indicator(state)
  *   cat_rates   [C], cat_props [C]    site_rate->getRate / getProp
  * Partial likelihoods live in device memory in "slots" chosen by the caller
- * (a PhyloNeighbor's partial_lh maps to slot (ptr - base) / block), stored
- * pattern-major [P][C][n] in the eigen basis, with one scale counter per
- * pattern (or per pattern and category in safe mode).
+ * (a PhyloNeighbor's partial_lh maps to slot (ptr - base) / block), in the
+ * eigen basis, with one scale counter per pattern (or per pattern and category
+ * in safe mode). The order of the values inside a slot is the engine's own;
+ * plk_read_partial gives them as [P][C][n].
  */
 #ifndef PLK_H
 #define PLK_H

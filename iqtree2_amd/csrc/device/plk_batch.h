@@ -365,8 +365,8 @@ struct XcdSplit {
 // The classes with protein in FP64 are held to 3 waves per SIMD (168
 // registers), the others of DNA and protein to 4, without spills in their
 // loops; the compiler's own choice left each one wave or more lower. Classes
-// of one storage have a fused kernel of their own: 90 partitions in FP32,
-// DNA and protein, 737 us fused in four waves, 878 in two launches.
+// of one storage have a fused kernel of their own (the tiles of 500 partitions:
+// FP64 2,940 us fused, 975 + 2,040 in two launches, FP32 2,880 and 645 + 2,130).
 template <int MASK>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(MASK & ~BC_ALL ? 1 : MASK & BC_PROT64 ? 3 : 4)))

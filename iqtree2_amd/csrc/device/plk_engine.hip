@@ -1725,9 +1725,12 @@ plk_status batch_fused(plk_context* ctx, const plk_batch_item* items, const int*
     // first calls each run one candidate (fused or per-class launches x 1,
     // 2, 4, 8 workgroups per CU) and time it; results do not depend on the
     // shape, so no call repeats work. Batches of fewer tiles than a few per
-    // CU keep the default: fused, as many workgroups as fit (90 partitions in
-    // FP32: 1071 us a call per class, two per CU; 938 fused). Likely-good shapes first,
-    // so exploring costs little.
+    // CU keep the default: fused, as many workgroups as fit. Against a launch per
+    // class at two per CU, all untuned: 500 partitions in FP64 3,490 and 4,040 us,
+    // 90 in FP32 930 and 984, 2 + 2 small ones (DNA, protein) 168 and 196 in FP64,
+    // 208 and 226 in FP32, of every class and storage 205 and 400. 200 of DNA
+    // alone: 247 and 208, until two per CU are tried. Likely-good shapes first, so
+    // exploring costs little.
     int lg = 0;
     while ((1 << lg) < total_tiles) lg++;
     const long key = (long)mix * 64 + lg;

@@ -138,7 +138,7 @@ __device__ inline ModelDev on_hbm(ModelDev m) {
 // side by side: [(S0, X0 X1), (S0, X2 X3), the same of S1, (X4, S0 S1)]
 // [lane p % 16 + 16 (x % 4)][2], so that a thread of its own (p, c) reads two
 // values at a time, too (a sweep of 20 taxa x 1,200 sites with the sixteens
-// side by side, one at a time: 2319 us, so: 2170; traversal 448 and 442 us).
+// side by side, one at a time: 2319 us, so: 2150; in [p][c][x] order 2120).
 template <typename T, int N, int C>
 struct Part {
     static constexpr bool kDna = N == 4, kProt = N == 20 && sizeof(T) == 8, kLanes = kDna && sizeof(T) == 8;

@@ -292,11 +292,10 @@ k_traverse_mfma(InstDev I, ModelDev m, const plk_op* __restrict__ ops, int nops,
 //     this one runs, and read from LDS, as is U^-1.
 // A wavefront owns a category; the only exchange is a mask of the patterns
 // that are below the rescale threshold in it, one barrier a step (normal mode).
-// 100 taxa x 20,000 patterns x 4 categories: 969 -> 448 us (3.1 TB/s with the
-// one slot in four re-read; 470 with waits for copies of children in flight,
-// 568 in 200 registers, two waves a SIMD; the protein
-// tiles of 500 partitions in a batch 3313 -> 2370 us). Bound now by the step's chain of products and
-// exchange, 2.2 us of a lone wavefront, at 2.4 wavefronts a SIMD.
+// 100 taxa x 19,792 patterns x 4 categories: 461 us, 1.63 GB to and from HBM
+// (3.5 TB/s), the 16x16x4 tile 969; of 500 partitions' protein tiles in a batch
+// 2,040 and 3,310. Bound by the step's chain of products and exchange, 2.2 us of
+// a lone wavefront, at 2.4 wavefronts a SIMD.
 constexpr int kProtPatterns = 32;          // of a wavefront
 
 // LDS: U^-1 | tip vectors and (1, 0, ...) for the root leaf, whose matrix holds
