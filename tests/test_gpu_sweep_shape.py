@@ -1,51 +1,35 @@
 """Workgroups of a device Newton pass: one a CU for a 4-state tree of up to four
 tiles a CU, else two, and as many as PLK_SWEEP_BLOCKS_PER_CU says where it is
-set, whatever the size; the lengths are those of the default."""
-import os
-import re
-import subprocess
-import sys
-
+set, whatever the size. A pass is reproducible to the bit with the same
+workgroups; with others its sums are added in another order."""
 import numpy as np
 import pytest
 
-from conftest import ROOT
+import iqtree2_amd as ia
+from test_gpu_parity import context_with
 
 pytestmark = pytest.mark.gpu
 
-# 8 categories: tiles of 32 patterns, about 400 of them (1.6 a CU)
-PROGRAM = """
-import sys
-sys.path.insert(0, %r)
-import iqtree2_amd as ia
-w = ia.Workload(seq_type=ia.DNA, ntaxa=20, nsite=13000, ncat=8, mean_len=0.3, seed=4)
-ctx = ia.Context(0)
-tree = ia.PhyloTree(ctx, w)
-lnl, _ = tree.optimize_all_branches(iterations=1, tolerance=1e-3, max_nr=100)
-print("tiles", -(-w.npatterns // 256) * 8, repr(lnl), *[repr(tree.get_length(a, b)) for a, b in tree.branches()])
-tree.close()
-ctx.close()
-"""
+
+def sweep(ctx, w):
+    tree = ia.PhyloTree(ctx, w)
+    lnl, n = tree.optimize_all_branches(iterations=1, tolerance=1e-3, max_nr=100)
+    out = np.array([lnl] + [tree.get_length(a, b) for a, b in tree.branches()])
+    tree.close()
+    return n, out
 
 
-def sweep(blocks):
-    env = dict(os.environ, PLK_SWEEP_TIMING="1")
-    env.pop("PLK_SWEEP_BLOCKS_PER_CU", None)
-    if blocks:
-        env["PLK_SWEEP_BLOCKS_PER_CU"] = str(blocks)
-    p = subprocess.run([sys.executable, "-c", PROGRAM % ROOT], env=env, capture_output=True, text=True, timeout=100)
-    assert p.returncode == 0, p.stderr
-    words = next(line for line in p.stdout.splitlines() if line.startswith("tiles")).split()
-    return (int(re.search(r"grid (\d+)", p.stderr).group(1)), int(words[1]), np.array([float(x) for x in words[2:]]))
-
-
-def test_workgroups_per_cu():
-    import torch
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    grid, tiles, values = sweep(None)
-    assert cus < tiles < 2 * cus
-    assert grid == cus
-    for blocks, expected in ((1, cus), (2, tiles)):
-        grid, _, other = sweep(blocks)
-        assert grid == expected, blocks
-        np.testing.assert_allclose(other, values, rtol=1e-9, atol=1e-12)
+def test_workgroups_per_cu(ctx):
+    # 8 categories: tiles of 32 patterns, 296 of them: more than one and fewer than two a CU
+    w = ia.Workload(seq_type=ia.DNA, ntaxa=20, nsite=13000, ncat=8, mean_len=0.3, seed=4)
+    assert 256 < w.npatterns / 32 < 512
+    n, values = sweep(ctx, w)
+    for blocks in (1, 2):
+        other = context_with({"PLK_SWEEP_BLOCKS_PER_CU": str(blocks)})
+        try:
+            m, got = sweep(other, w)
+        finally:
+            other.close()
+        assert m == n
+        np.testing.assert_allclose(got, values, rtol=1e-9, atol=1e-12)
+        assert np.array_equal(got, values) == (blocks == 1)
